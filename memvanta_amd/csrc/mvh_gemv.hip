@@ -379,48 +379,6 @@ __global__ __launch_bounds__(kGemvThreads) void gemv_f32act_tokens_kernel(const 
     }
 }
 
-// Default batched prefill numerics (q4_row_batch4_fp32 / q8_row_batch4_fp32,
-// src/gguf_kernels.cpp:191-209; batch8 = two batch4, :211-216): per
-// (row, token) eight lane accumulators run over ALL blocks without reset,
-// term = fma(float(q)*d, x, acc) with the product float(q)*d rounded first;
-// result = t0+t1+..+t7.  One thread per (row, token); blockIdx.y = token.
-template <uint32_t TYPE>
-__global__ __launch_bounds__(256) void batch4_f32act_kernel(const uint8_t* __restrict__ W,
-                                                             const float* __restrict__ x, float* __restrict__ y,
-                                                             int N, int nb) {
-    constexpr int BB = Blk<TYPE>::kBytes;
-    extern __shared__ __align__(16) float s_xt[];
-    const int K = nb * 32;
-    const float* xt = x + static_cast<size_t>(blockIdx.y) * K;
-    for (int c = threadIdx.x; c < K / 4; c += blockDim.x)
-        reinterpret_cast<float4*>(s_xt)[c] = reinterpret_cast<const float4*>(xt)[c];
-    __syncthreads();
-    const int r = blockIdx.x * blockDim.x + threadIdx.x;
-    if (r >= N) return;
-    const uint8_t* rowp = W + static_cast<size_t>(r) * nb * BB;
-    float t[8];
-#pragma unroll
-    for (int j = 0; j < 8; ++j) t[j] = 0.0f;
-    for (int b = 0; b < nb; ++b) {
-        const uint16_t* src = reinterpret_cast<const uint16_t*>(rowp + static_cast<size_t>(b) * BB);
-        uint32_t qs[Blk<TYPE>::kQdw];
-#pragma unroll
-        for (int k = 0; k < Blk<TYPE>::kQdw; ++k)
-            qs[k] = src[1 + 2 * k] | (static_cast<uint32_t>(src[2 + 2 * k]) << 16);
-        const float d = h2f(src[0]);
-        const float* xb = s_xt + b * 32;
-#pragma unroll
-        for (int e = 0; e < 32; ++e) {
-            const float q = static_cast<float>(Blk<TYPE>::value(qs, e)) * d;
-            t[e & 7] = fmaf(q, xb[e], t[e & 7]);
-        }
-    }
-    float s = t[0];
-#pragma unroll
-    for (int j = 1; j < 8; ++j) s = s + t[j];
-    y[static_cast<size_t>(blockIdx.y) * N + r] = s;
-}
-
 // dot_q8_0_fp32 / dot_q4_0_fp32 per row (tensor_matvec's Q8_0 branch and the
 // fp32-activation Q4_0 dot, src/gguf_kernels.cpp:93-120) for one token, K %
 // 256 == 0, K / 256 <= 64, in the structure of the persistent Q4_0 x Q8 GEMV:
@@ -575,189 +533,6 @@ __global__ __launch_bounds__(256) void gemv_f32act_persistent_nq8_0(
     gemv_f32act_persistent<kNQ8_0, 4>(W, x, y, N, nb, ntiles);
 }
 
-// The same numerics for K % 256 == 0 with the work spread over lanes: lane
-// (row, j) owns accumulator j of its row for kBT tokens, i.e. elements j,
-// j+8, j+16, j+24 of every block in that order (the reference's 8-wide
-// vector lane j); eight lanes per row, eight rows per wave, 32 rows per
-// workgroup.  Each dequantized float(q)*d feeds the kBT tokens' fmas.  The
-// weights come in 8-block units (16-byte loads; the eight lanes of a row load
-// the same bytes); the activations of the kBT tokens come through LDS one
-// 8-block chunk at a time, stored as [token][block][j][m] so lane j reads its
-// four elements x[32b + j + 8m] with one 16-byte read.  The final
-// t0 + t1 + ... + t7 runs in order through LDS.
-constexpr int kBT = 8;         // tokens per workgroup
-constexpr int kBRows = 32;     // rows per workgroup
-constexpr int kBChunk = 256;   // activation elements per LDS chunk (one 8-block unit)
-
-template <uint32_t TYPE>
-struct Unit;
-template <>
-struct Unit<kQ4_0> {
-    static constexpr int kU4 = 9;  // 16-byte loads per 8 blocks (144 bytes)
-    // block jb of the unit: f16 scale bits and the 16 quant bytes as 4 dwords
-    static __device__ __forceinline__ void block(const uint32_t (&w)[4 * kU4], int jb, uint32_t& dbits,
-                                                 uint32_t (&qs)[4]) {
-        const int o = 18 * jb;
-        if ((jb & 1) == 0) {
-            dbits = w[o / 4] & 0xffffu;
-#pragma unroll
-            for (int k = 0; k < 4; ++k) qs[k] = align16(w[o / 4 + k + 1], w[o / 4 + k]);
-        } else {
-            dbits = w[o / 4] >> 16;
-#pragma unroll
-            for (int k = 0; k < 4; ++k) qs[k] = w[(o + 2) / 4 + k];
-        }
-    }
-    // elements j, j+8, j+16, j+24: low nibbles of bytes j, 8+j, high nibbles of the same
-    static __device__ __forceinline__ void lane_values(const uint32_t (&qs)[4], int j, int (&v)[4]) {
-        const uint32_t sh = 8u * static_cast<uint32_t>(j & 3);
-        const uint32_t b0 = ((j & 4) ? qs[1] : qs[0]) >> sh, b1 = ((j & 4) ? qs[3] : qs[2]) >> sh;
-        v[0] = static_cast<int>(b0 & 15u) - 8;
-        v[1] = static_cast<int>(b1 & 15u) - 8;
-        v[2] = static_cast<int>((b0 >> 4) & 15u) - 8;
-        v[3] = static_cast<int>((b1 >> 4) & 15u) - 8;
-    }
-};
-template <>
-struct Unit<kQ8_0> {
-    static constexpr int kU4 = 17;  // 272 bytes
-    static __device__ __forceinline__ void block(const uint32_t (&w)[4 * kU4], int jb, uint32_t& dbits,
-                                                 uint32_t (&qs)[8]) {
-        const int o = 34 * jb;
-        if ((jb & 1) == 0) {
-            dbits = w[o / 4] & 0xffffu;
-#pragma unroll
-            for (int k = 0; k < 8; ++k) qs[k] = align16(w[o / 4 + k + 1], w[o / 4 + k]);
-        } else {
-            dbits = w[o / 4] >> 16;
-#pragma unroll
-            for (int k = 0; k < 8; ++k) qs[k] = w[(o + 2) / 4 + k];
-        }
-    }
-    // elements j + 8m: byte j + 8m of the 32 int8 values
-    static __device__ __forceinline__ void lane_values(const uint32_t (&qs)[8], int j, int (&v)[4]) {
-        const uint32_t sh = 8u * static_cast<uint32_t>(j & 3);
-#pragma unroll
-        for (int m = 0; m < 4; ++m)
-            v[m] = static_cast<int>(static_cast<int8_t>(((j & 4) ? qs[2 * m + 1] : qs[2 * m]) >> sh));
-    }
-};
-
-template <uint32_t TYPE>
-__global__ __launch_bounds__(256) void batch_f32act_lanes_kernel(const uint8_t* __restrict__ W,
-                                                                 const float* __restrict__ x, float* __restrict__ y,
-                                                                 int N, int nb) {
-    using U = Unit<TYPE>;
-    constexpr int kQdw = Blk<TYPE>::kQdw;
-    __shared__ __align__(16) float s_x[2][kBT * kBChunk];  // [token][block][j][m], double-buffered
-    const int t = threadIdx.x, j = t & 7;
-    const int rl = t >> 3;  // row within the workgroup
-    const int r = blockIdx.x * kBRows + rl;
-    const int tok0 = blockIdx.y * kBT;
-    const int K = nb * 32, units = nb / 8;
-    const size_t row_bytes = static_cast<size_t>(nb) * Blk<TYPE>::kBytes;
-    const uint4* wrow = reinterpret_cast<const uint4*>(W + static_cast<size_t>(min(r, N - 1)) * row_bytes);
-
-    // chunk c of the kBT activation rows: 2 float4 per thread (kBT * 256
-    // floats) into registers, written to LDS after the current unit's fmas,
-    // so the wait for them neither delays those fmas nor covers the weight
-    // loads issued after them
-    constexpr int kSt = kBT * kBChunk / 4 / 256;
-    auto stage_load = [&](int c, float4 (&v)[kSt]) {
-#pragma unroll
-        for (int k = 0; k < kSt; ++k) {
-            const int f = t + 256 * k;  // float4 index within the chunk: token f / 64, element 4 (f % 64)
-            v[k] = *reinterpret_cast<const float4*>(x + static_cast<size_t>(tok0 + (f >> 6)) * K + c * kBChunk +
-                                                    4 * (f & 63));
-        }
-    };
-    auto stage_store = [&](const float4 (&v)[kSt], int buf) {
-#pragma unroll
-        for (int k = 0; k < kSt; ++k) {
-            const int f = t + 256 * k;
-            const int tk = f >> 6, e = 4 * (f & 63);
-            const float vv[4] = {v[k].x, v[k].y, v[k].z, v[k].w};
-#pragma unroll
-            for (int i = 0; i < 4; ++i) {  // element e+i: block (e+i)/32, lane (e+i)%8, m = ((e+i)%32)/8
-                const int ei = e + i;
-                s_x[buf][((tk * 8 + (ei >> 5)) * 8 + (ei & 7)) * 4 + ((ei & 31) >> 3)] = vv[i];
-            }
-        }
-    };
-
-    float acc[kBT];
-#pragma unroll
-    for (int k = 0; k < kBT; ++k) acc[k] = 0.0f;
-    uint32_t w[4 * U::kU4];
-    auto load = [&](int u) {
-#pragma unroll
-        for (int k = 0; k < U::kU4; ++k) {
-            const uint4 v = wrow[u * U::kU4 + k];
-            w[4 * k] = v.x;
-            w[4 * k + 1] = v.y;
-            w[4 * k + 2] = v.z;
-            w[4 * k + 3] = v.w;
-        }
-    };
-    float4 xs[kSt];
-    stage_load(0, xs);
-    load(0);
-    stage_store(xs, 0);
-    __syncthreads();
-    for (int u = 0; u < units; ++u) {
-        const int buf = u & 1;
-        // the next unit's loads and staging run unconditionally (the last
-        // unit reloads itself and restages into the idle buffer), so no
-        // branch lets the compiler move the staging stores ahead of the fmas
-        const int nu = min(u + 1, units - 1);
-        uint32_t cur[4 * U::kU4];
-#pragma unroll
-        for (int k = 0; k < 4 * U::kU4; ++k) cur[k] = w[k];
-        stage_load(nu, xs);
-        load(nu);
-#pragma unroll
-        for (int jb = 0; jb < 8; ++jb) {
-            uint32_t dbits, qs[kQdw];
-            U::block(cur, jb, dbits, qs);
-            const float d = h2f(dbits);
-            int v[4];
-            U::lane_values(qs, j, v);
-            float q[4];
-#pragma unroll
-            for (int m = 0; m < 4; ++m) q[m] = static_cast<float>(v[m]) * d;
-#pragma unroll
-            for (int k = 0; k < kBT; ++k) {
-                const float4 xv = *reinterpret_cast<const float4*>(&s_x[buf][((k * 8 + jb) * 8 + j) * 4]);
-                acc[k] = fmaf(q[0], xv.x, acc[k]);
-                acc[k] = fmaf(q[1], xv.y, acc[k]);
-                acc[k] = fmaf(q[2], xv.z, acc[k]);
-                acc[k] = fmaf(q[3], xv.w, acc[k]);
-            }
-            // each block's LDS reads stay with its fmas, and the staging
-            // stores stay after the last block: hoisted, the reads take a
-            // register set per block and the stores wait for the activation
-            // loads in the middle of the fmas
-            __builtin_amdgcn_sched_barrier(0);
-        }
-        stage_store(xs, buf ^ 1);  // s_x[buf ^ 1] was last read by unit u - 1
-        __syncthreads();  // s_x[buf ^ 1] is complete; s_x[buf] is free for unit u + 2
-    }
-    // t0 + t1 + ... + t7 per (row, token), in order, through LDS
-    float* s_red = &s_x[0][0];  // [row][token][j]
-#pragma unroll
-    for (int k = 0; k < kBT; ++k) s_red[(rl * kBT + k) * 8 + j] = acc[k];
-    __syncthreads();
-    {
-        const int tk = t / kBRows, row = t % kBRows;  // one output per thread, rows fastest
-        const float* p = s_red + (row * kBT + tk) * 8;
-        float sum = p[0];
-#pragma unroll
-        for (int i = 1; i < 8; ++i) sum = sum + p[i];
-        const int orow = blockIdx.x * kBRows + row;
-        if (orow < N) y[static_cast<size_t>(tok0 + tk) * N + orow] = sum;
-    }
-}
-
 // q4/q8_row_batch4_fp32 numerics (src/gguf_kernels.cpp:191-216) for Q4_0 and
 // Q8_0 with K % 256 == 0, each activation read feeding two rows: lane (row
 // pair, j) owns accumulator j of two rows for kR2T tokens, elements j, j+8,
@@ -784,6 +559,7 @@ __global__ __launch_bounds__(256) void batch_f32act_lanes_kernel(const uint8_t* 
 // t carries the chains of (row, token) t and t + 256 over the unit's eight
 // blocks.  The activation blocks are padded to 36 floats in LDS so the eight
 // blocks of a token fall in different banks.
+constexpr int kBChunk = 256;  // activation elements per LDS chunk (one 8-block unit)
 constexpr int kR2T = 8;       // tokens per thread (16 measured slower: 214 VGPRs, half the workgroups)
 constexpr int kR2Rows = 32;   // rows per workgroup
 constexpr int kR2Tok = 2 * kR2T;
@@ -1496,47 +1272,6 @@ hipError_t launch_gemv_native_f32act(uint32_t type, const uint8_t* W, const floa
     if (type == kNQ4_0) return launch_f32act_any<kNQ4_0>(W, x, y, rows, cols, batch, st);
     if (type == kNQ8_0) return launch_f32act_any<kNQ8_0>(W, x, y, rows, cols, batch, st);
     return hipErrorInvalidValue;
-}
-
-hipError_t launch_batch4_f32act(uint32_t type, const uint8_t* W, const float* x, float* y, size_t rows, size_t cols,
-                                size_t batch, hipStream_t st) {
-    if (!rows || !batch) return hipSuccess;
-    const int nb = static_cast<int>(cols / 32);
-    static_assert(kBT * kBRows == 256, "one output per thread in the final sum");
-    if (cols % 256 == 0 && batch >= kR2Tok) {
-        // whole groups of kR2Tok tokens with two rows per lane, the rest below
-        const size_t groups = batch / kR2Tok;
-        const dim3 grid(static_cast<unsigned>((rows + kR2Rows - 1) / kR2Rows), static_cast<unsigned>(groups));
-        if (type == kQ4_0)
-            batch_f32act_rows2_kernel<kQ4_0, false><<<grid, 256, 0, st>>>(W, x, y, static_cast<int>(rows), nb);
-        else
-            batch_f32act_rows2_kernel<kQ8_0, false><<<grid, 256, 0, st>>>(W, x, y, static_cast<int>(rows), nb);
-        const size_t done = groups * kR2Tok;
-        if (done == batch) return hipGetLastError();
-        x += done * cols;
-        y += done * rows;
-        batch -= done;
-    }
-    if (cols % 256 == 0 && batch >= kBT) {
-        // whole groups of kBT tokens on the lane-spread kernel, the rest per token below
-        const size_t groups = batch / kBT;
-        const dim3 grid(static_cast<unsigned>((rows + kBRows - 1) / kBRows), static_cast<unsigned>(groups));
-        if (type == kQ4_0)
-            batch_f32act_lanes_kernel<kQ4_0><<<grid, 256, 0, st>>>(W, x, y, static_cast<int>(rows), nb);
-        else
-            batch_f32act_lanes_kernel<kQ8_0><<<grid, 256, 0, st>>>(W, x, y, static_cast<int>(rows), nb);
-        const size_t done = groups * kBT;
-        if (done == batch) return hipGetLastError();
-        x += done * cols;
-        y += done * rows;
-        batch -= done;
-    }
-    const dim3 grid(static_cast<unsigned>((rows + 255) / 256), static_cast<unsigned>(batch));
-    if (type == kQ4_0)
-        batch4_f32act_kernel<kQ4_0><<<grid, 256, cols * sizeof(float), st>>>(W, x, y, static_cast<int>(rows), nb);
-    else
-        batch4_f32act_kernel<kQ8_0><<<grid, 256, cols * sizeof(float), st>>>(W, x, y, static_cast<int>(rows), nb);
-    return hipGetLastError();
 }
 
 hipError_t launch_gemv_f32(const float* W, const float* x, float* y, size_t rows, size_t cols, size_t batch,

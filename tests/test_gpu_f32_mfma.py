@@ -1,0 +1,31 @@
+"""The batched fp32-activation products on the f32 matrix pipe (memvanta_amd/csrc/mvh_gemm_f32.hip): bit-exact
+against the oracle at the edges of their tiles.
+
+Both numerics are fma chains in a fixed order and the kernels run the same chains, so the tolerance is none."""
+import numpy as np
+import pytest
+
+from conftest import assert_bitexact
+from memvanta_amd import capi, synth
+
+pytestmark = pytest.mark.gpu
+
+
+def _case(rng, ty, n, k, batch):
+    w = synth.quantize(ty, rng.standard_normal((n, k), dtype=np.float32) * np.float32(0.02)).reshape(-1)
+    return w, synth.activations(rng, batch, k)
+
+
+# rows / tokens: one, just below, at and past the 16 / 32 / 48-row and 16 / 32-token tiles; K: one block, one unit less
+# or more than whole 8-block units (the 2-byte staging), two units and the shortest whole unit (no next unit to fetch)
+@pytest.mark.parametrize("ty", [synth.Q4_0, synth.Q8_0])
+@pytest.mark.parametrize("batch,k,n", [(4, 32, 1), (16, 288, 17), (20, 224, 33), (4, 256, 15), (36, 512, 49),
+                                       (68, 768, 31), (28, 1024, 4096), (12, 1280, 16400), (100, 256, 8200),
+                                       (512, 256, 100), (32, 256, 11008)])
+def test_chain_tiles_bitexact(ctx, oracle, ty, batch, k, n):
+    rng = np.random.default_rng(batch * 3 + k + n + ty)
+    w, x = _case(rng, ty, n, k, batch)
+    t = ctx.upload("blk.0.attn_q.weight", ty, k, n, w)
+    got = ctx.matmul_batch_v06(t, x, capi.MVH_ACT_REF)
+    assert_bitexact(got, oracle.matmul_batch_v06(w, ty, n, k, x, is_ffn=False, force_q8=False), f"B={batch} K={k} N={n}")
+    t.free()

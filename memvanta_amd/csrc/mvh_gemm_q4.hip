@@ -190,173 +190,202 @@ __global__ __launch_bounds__(64) void gemm_q4_0_q8_mfma_kernel(const uint8_t* __
     }
 }
 
-// The same numerics with a workgroup of 4 waves sharing one LDS copy of each
-// K-chunk: 64 weight rows (wave w computes rows 16w .. 16w+15) x 16*TG
-// tokens.  The chunk's raw weights (64 rows x 144 B), activation operands (TG
-// x 4 KB, operand order) and scales come in with 16-byte loads one chunk
-// ahead into registers, go to the idle half of a double-buffered LDS copy
-// after the current chunk's compute, and one workgroup barrier per chunk
-// hands them over; the staging also copies each row's f16 block scales to a
-// [block][row] table.  The weights are the MFMA's A operand, so a lane holds
-// rows 4h .. 4h+3 of one token (li) and reads, per block, four row scales
-// (8 bytes) and one activation scale per token group; C = (-8) x A for the
-// next block is issued before the current block's sums are used.  Against
-// the wave-private kernel: no register ring of activation operands (about
-// half the VGPRs, twice the resident waves), a quarter of the activation
-// traffic and a third of the LDS bytes per block.
-template <int TG>
-__global__ __launch_bounds__(256) void gemm_q4_0_q8_mfma_wg_kernel(const uint8_t* __restrict__ W,
-                                                                   const int8_t* __restrict__ aq,
-                                                                   const float* __restrict__ ad,
-                                                                   float* __restrict__ y, int N, int nb, int B) {
-    constexpr int kToks = 16 * TG;
-    constexpr int kWgRows = 64;
-    constexpr int kRaw = kWgRows * kUnit;        // 9216 bytes of raw weights per chunk
-    constexpr int kPieces = kRaw / 16;           // 576
-    constexpr int kWLd = (kPieces + 255) / 256;  // 3 weight loads per thread
-    constexpr int kA = TG * 4096;                // activation operand bytes per chunk
-    constexpr int kDa = kChunk * kToks;          // activation scales per chunk
-    __shared__ __align__(16) uint8_t s_raw[2][kRaw + 16];                // + a spare slot for unused stores
-    __shared__ __align__(16) uint16_t s_dw[2][kChunk * kWgRows + 8];      // [block][row] f16 scales + spare
-    __shared__ __align__(16) int8_t s_a[2][kA];
-    __shared__ __align__(16) float s_da[2][kDa];                          // [block][token]
+typedef int v16i __attribute__((ext_vector_type(16)));
+typedef float v16f __attribute__((ext_vector_type(16)));
+typedef float v32f __attribute__((ext_vector_type(32)));
 
-    const int t = threadIdx.x, l = t & 63, wv = t >> 6, li = l & 15, h = l >> 4;
+// 12582912 = 1.5 * 2^23: an int32 sum s (|s| < 2^22) added to this float's bits
+// gives the float 12582912 + s.
+constexpr int kMagic = 0x4B400000;
+
+// The same numerics for large batches: a workgroup of 4 waves shares one LDS
+// copy of each K-step of 4 blocks, and a wave computes 32 tokens x 32 rows
+// (WT waves over the tokens, 4 / WT over the rows).  Per block and 32 x 32
+// outputs:
+//   * one v_mfma_i32_32x32x32_i8 (twice the rate of the 16x16x32 form) of the
+//     activations and 16 (q - 8), a nibble in a byte's upper half with its top
+//     bit flipped; no extra product for the -8;
+//   * its accumulator starts at kMagic, so the result is the float 12582912 +
+//     16 isum, and fma(that, 1/16, -12582912/16) = float(isum) exactly: a
+//     v_cvt_f32_i32 issues at half the rate of an fma;
+//   * f16(d_w) * d_a for two blocks and all 32 x 32 outputs is one rank-one
+//     v_mfma_f32_32x32x1_2b_f32, each product rounded once as the reference's.
+// The fmas of a block run while its successor's operands are read, and the
+// successor's products then take their registers.
+// What bounds it: VALU and f32-MFMA issue, which exclude each other (per 16 x
+// 16 outputs and block about 20 cycles of fma, 8 + 8 of MFMA, 7 of unpacking),
+// at two waves per SIMD.  Masks and constants are held in VGPRs: an operand in
+// an SGPR halves a VALU instruction's rate (4.4 against 2.5 cycles measured).
+// Against the four-wave 16x16x32 kernel it replaces, both with the quantizer:
+// 512 tokens 4096x4096 61 -> 43 us, 4096->11008 138 -> 97, 11008->4096 140 ->
+// 97, 4096->22016 260 -> 176 (525 TOP/s).
+template <int WT>
+__global__ __launch_bounds__(256, 2) void gemm_q4_0_q8_tile_kernel(const uint8_t* __restrict__ W,
+                                                                const int8_t* __restrict__ aq,
+                                                                const float* __restrict__ ad,
+                                                                float* __restrict__ y, int N, int nb, int B) {
+    constexpr int kStep = 4;              // blocks per K-step
+    constexpr int kBytes = 18 * kStep;    // a row's bytes of a step
+    constexpr int kPitch = kBytes + 4;    // an odd number of dwords: 32 rows on 32 banks
+    constexpr int WR = 4 / WT;            // waves over the rows
+    constexpr int kToks = 32 * WT, kWgRows = 32 * WR;
+    constexpr int kPieces = kWgRows * 9;
+    constexpr int kWLd = (kPieces + 255) / 256;  // 8-byte weight loads per thread
+    constexpr int kAu = WT;                      // activation units per thread
+    constexpr int kDl = (kToks * kStep + 255) / 256;
+    __shared__ __align__(16) uint8_t s_w[2][kWgRows * kPitch + 16];     // + a spare slot for unused stores
+    __shared__ __align__(16) int8_t s_a[2][kStep * 2 * kToks * 16];     // [block][half][token][16]
+    __shared__ __align__(16) float s_da[2][kStep * kToks];              // [block][token]
+
+    const int t = threadIdx.x, l = t & 63, wv = __builtin_amdgcn_readfirstlane(t >> 6), li = l & 31, h = l >> 5;
+    const int wt = wv % WT, wr = wv / WT;
     const int r0 = blockIdx.x * kWgRows, t0 = blockIdx.y * kToks;
     const size_t row_bytes = static_cast<size_t>(nb) * 18, K = static_cast<size_t>(nb) * 32;
-    const int nchunks = nb / kChunk;
+    const int steps = nb / kStep;
 
-    // weight piece p = t + 256 i: row p / 9, unit bytes 16 (p % 9); piece k < 8 of a
-    // row holds block k's scale at its byte 2k
-    const uint8_t* wsrc[kWLd];
-    int wdst[kWLd], sdst[kWLd], sdw[kWLd];
+    const uint8_t* wbase = W + static_cast<size_t>(r0) * row_bytes;
+    uint32_t wsrc[kWLd];
+    int wdst[kWLd];
 #pragma unroll
     for (int i = 0; i < kWLd; ++i) {
-        const int p = t + 256 * i, pc = min(p, kPieces - 1), k = pc % 9;
-        wsrc[i] = W + static_cast<size_t>(min(r0 + pc / 9, N - 1)) * row_bytes + k * 16;
-        wdst[i] = p < kPieces ? (pc / 9) * kUnit + k * 16 : kRaw;
-        sdst[i] = p < kPieces && k < 8 ? k * kWgRows + pc / 9 : kChunk * kWgRows;
-        sdw[i] = k & 7;  // the scale's halfword within the piece
+        const int p = t + 256 * i, pc = min(p, kPieces - 1), row = pc / 9, k = pc % 9;
+        wsrc[i] = static_cast<uint32_t>(min(row, N - 1 - r0)) * static_cast<uint32_t>(row_bytes) + k * 8;
+        wdst[i] = p < kPieces ? row * kPitch + k * 8 : kWgRows * kPitch;
     }
-    const int8_t* asrc[TG];
+    // activation unit u = t + 256 i: token u % 16 of 16-token slab u / 128, half u / 16 % 2 (its
+    // quarters q and q + 2, as a weight byte's two nibbles) of block u / 32 % 4; slabs past the
+    // last read the last one (not stored)
+    const int slab0 = static_cast<int>(blockIdx.y) * 2 * WT, slabs = (B + 15) / 16;
+    const int8_t* const abase = aq + static_cast<size_t>(slab0) * 16 * K;
+    uint32_t asrc[kAu];
 #pragma unroll
-    for (int g = 0; g < TG; ++g)
-        asrc[g] = aq + static_cast<size_t>(min(blockIdx.y * TG + g, (B - 1) / 16)) * 16 * K + 16 * t;
-    // scale e = t + 256 i: token e / 8, block e % 8 (TG = 1: threads t, t + 128 load the same scale)
-    constexpr int kDL = (kDa + 255) / 256;
-    const float* dsrc[kDL];
-    int ddst[kDL];
+    for (int i = 0; i < kAu; ++i)
+        asrc[i] = static_cast<uint32_t>(min(2 * i + (t >> 7), slabs - 1 - slab0)) * static_cast<uint32_t>(16 * K) +
+                  (t >> 5 & 3) * 512 + (t >> 4 & 1) * 128 + (t & 15) * 8;
+    const int adst = (t >> 4 & 7) * (kToks * 16) + ((t >> 7) * 16 + (t & 15)) * 16;
+    // scale e = t + 256 i: token e / 4, block e % 4
+    const float* const dbase = ad + static_cast<size_t>(t0) * nb;
+    uint32_t dsrc[kDl];
+    int ddst[kDl];
 #pragma unroll
-    for (int i = 0; i < kDL; ++i) {
-        const int e = (t + 256 * i) % kDa, d_tok = e / 8, d_blk = e % 8;
-        dsrc[i] = ad + static_cast<size_t>(min(t0 + d_tok, B - 1)) * nb + d_blk;
-        ddst[i] = d_blk * kToks + d_tok;
+    for (int i = 0; i < kDl; ++i) {
+        const int e = (t + 256 * i) % (kToks * kStep);
+        dsrc[i] = static_cast<uint32_t>(min(e / 4, B - 1 - t0)) * static_cast<uint32_t>(nb) + e % 4;
+        ddst[i] = e % 4 * kToks + e / 4;
     }
 
-    uint4 wreg[kWLd];
-    uint4 areg[TG];
-    float dreg[kDL];
-    auto load = [&](int c) {
-        const size_t wc = static_cast<size_t>(c) * kUnit;
+    struct Regs {
+        uint2 w[kWLd], a[kAu][2];
+        float d[kDl];
+    } q;
+    auto load = [&](int c) __attribute__((always_inline)) {
+        const uint8_t* wc = wbase + static_cast<size_t>(c) * kBytes;
 #pragma unroll
-        for (int i = 0; i < kWLd; ++i) wreg[i] = ld_global16(wsrc[i] + wc);
+        for (int i = 0; i < kWLd; ++i) q.w[i] = ld_global8(wc + wsrc[i]);
 #pragma unroll
-        for (int g = 0; g < TG; ++g) areg[g] = ld_global16(asrc[g] + static_cast<size_t>(c) * 4096);
-#pragma unroll
-        for (int i = 0; i < kDL; ++i) dreg[i] = dsrc[i][c * kChunk];
-    };
-    auto store = [&](int buf) {
-#pragma unroll
-        for (int i = 0; i < kWLd; ++i) {
-            *reinterpret_cast<uint4*>(&s_raw[buf][wdst[i]]) = wreg[i];
-            // halfword sdw[i] of the piece (dword sdw / 2, half sdw % 2)
-            const bool upper = (sdw[i] & 4) != 0;
-            const uint32_t d0 = upper ? wreg[i].z : wreg[i].x, d1 = upper ? wreg[i].w : wreg[i].y;
-            const uint32_t dd = (sdw[i] & 2) ? d1 : d0;
-            s_dw[buf][sdst[i]] = static_cast<uint16_t>(dd >> (16 * (sdw[i] & 1)));
+        for (int i = 0; i < kAu; ++i) {
+            q.a[i][0] = ld_global8(abase + static_cast<size_t>(c) * 2048 + asrc[i]);
+            q.a[i][1] = ld_global8(abase + static_cast<size_t>(c) * 2048 + 256 + asrc[i]);
         }
 #pragma unroll
-        for (int g = 0; g < TG; ++g) *reinterpret_cast<uint4*>(&s_a[buf][g * 4096 + 16 * t]) = areg[g];
+        for (int i = 0; i < kDl; ++i) q.d[i] = (dbase + c * kStep)[dsrc[i]];
+    };
+    auto store = [&](int buf) __attribute__((always_inline)) {
 #pragma unroll
-        for (int i = 0; i < kDL; ++i) s_da[buf][ddst[i]] = dreg[i];
+        for (int i = 0; i < kWLd; ++i) {
+            uint32_t* p = reinterpret_cast<uint32_t*>(s_w[buf] + wdst[i]);
+            p[0] = q.w[i].x, p[1] = q.w[i].y;
+        }
+#pragma unroll
+        for (int i = 0; i < kAu; ++i)
+            *reinterpret_cast<uint4*>(s_a[buf] + adst + i * 512) = make_uint4(q.a[i][0].x, q.a[i][0].y, q.a[i][1].x, q.a[i][1].y);
+#pragma unroll
+        for (int i = 0; i < kDl; ++i) s_da[buf][ddst[i]] = q.d[i];
     };
 
-    float acc[TG][4];
+    v16f acc = {};
+    v16i is[2];
+    v32f p = {};
+    v16i magic;
 #pragma unroll
-    for (int g = 0; g < TG; ++g) acc[g][0] = acc[g][1] = acc[g][2] = acc[g][3] = 0.f;
-    // the lane's weight operand bytes: row 16 wv + li, qs[8(h&1) .. +8) of each block, nibble half h >> 1
-    const int my_row = (16 * wv + li) * kUnit;
-    const uint32_t nib_shift = 4u * static_cast<uint32_t>(h >> 1);
+    for (int i = 0; i < 16; ++i) magic[i] = kMagic;
+    is[0] = is[1] = magic;
+    // in VGPRs: see above
+    uint32_t mask = 0xf0f0f0f0u, bias = 0x80808080u;
+    float sixteenth = 0.0625f, off = -12582912.0f / 16.0f;
+    asm volatile("" : "+v"(mask), "+v"(bias), "+v"(sixteenth), "+v"(off));
+    const int my_w = (32 * wr + li) * kPitch, my_a = (h * kToks + 32 * wt + li) * 16, my_d = 32 * wt + li;
+
+    struct Ops {
+        v4i a[2];
+        uint32_t q[2][3], d;
+        float da;
+    };
+    auto read = [&](int buf, int j, Ops& o) __attribute__((always_inline)) {  // blocks j and j + 1, j even: 18j is a whole dword
+        const uint8_t* w = s_w[buf] + my_w + 18 * j;
+        o.d = *reinterpret_cast<const uint16_t*>(w + 18 * h);
+        o.da = s_da[buf][(j + h) * kToks + my_d];
+        const uint32_t* p0 = reinterpret_cast<const uint32_t*>(w + 8 * h);
+        o.q[0][0] = p0[0], o.q[0][1] = p0[1], o.q[0][2] = p0[2];
+        const uint32_t* p1 = reinterpret_cast<const uint32_t*>(w + 20 + 8 * h);
+        o.q[1][0] = p1[0], o.q[1][1] = p1[1];
+#pragma unroll
+        for (int b = 0; b < 2; ++b)
+            o.a[b] = *reinterpret_cast<const v4i*>(s_a[buf] + (j + b) * (2 * kToks * 16) + my_a);
+    };
+    auto chain = [&](int b) __attribute__((always_inline)) {
+#pragma unroll
+        for (int i = 0; i < 16; ++i) {
+            const float s = fmaf(__int_as_float(is[b][i]), sixteenth, off);
+            acc[i] = fmaf(p[16 * b + i], s, acc[i]);
+        }
+    };
+    auto operand = [&](uint32_t q0, uint32_t q1) __attribute__((always_inline)) {
+        return v4i{static_cast<int>((q0 << 4 & mask) ^ bias), static_cast<int>((q1 << 4 & mask) ^ bias),
+                   static_cast<int>((q0 & mask) ^ bias), static_cast<int>((q1 & mask) ^ bias)};
+    };
+    auto pair = [&](const Ops& o) __attribute__((always_inline)) {
+        const v4i w0 = operand(align16(o.q[0][1], o.q[0][0]), align16(o.q[0][2], o.q[0][1]));
+        const float dw = h2f(o.d);
+        chain(0);
+        __builtin_amdgcn_sched_barrier(0);
+        is[0] = __builtin_amdgcn_mfma_i32_32x32x32_i8(o.a[0], w0, magic, 0, 0, 0);
+        const v4i w1 = operand(o.q[1][0], o.q[1][1]);
+        chain(1);
+        __builtin_amdgcn_sched_barrier(0);
+        is[1] = __builtin_amdgcn_mfma_i32_32x32x32_i8(o.a[1], w1, magic, 0, 0, 0);
+        p = __builtin_amdgcn_mfma_f32_32x32x1f32(o.da, dw, v32f{}, 0, 0, 0);
+        __builtin_amdgcn_sched_barrier(0);
+    };
 
     load(0);
     store(0);
-    __syncthreads();
-    for (int c = 0; c < nchunks; ++c) {
-        const int buf = c & 1;
-        load(min(c + 1, nchunks - 1));  // unconditional: the last chunk reloads itself
-        const uint8_t* my_q = &s_raw[buf][my_row + 2 + 8 * (h & 1)];
-        long a_cur[TG];
-        v4i c8_cur[TG];
+    load(min(1, steps - 1));
+    for (int c = 0; c < steps; c += 2) {
 #pragma unroll
-        for (int g = 0; g < TG; ++g) {
-            a_cur[g] = *reinterpret_cast<const long*>(&s_a[buf][g * 4096 + 8 * l]);
-            c8_cur[g] = __builtin_amdgcn_mfma_i32_16x16x32_i8(kMinus8, a_cur[g], v4i{0, 0, 0, 0}, 0, 0, 0);
+        for (int d = 0; d < 2; ++d) {
+            __syncthreads();
+            Ops o;
+            read(d, 0, o);
+            __builtin_amdgcn_sched_barrier(0);
+            pair(o);
+            read(d, 2, o);
+            store(d ^ 1);  // the idle buffer was last read in step c + d - 1
+            load(min(c + d + 2, steps - 1));  // unconditional: past the end the last step again
+            __builtin_amdgcn_sched_barrier(0);
+            pair(o);
         }
-#pragma unroll
-        for (int j = 0; j < kChunk; ++j) {
-            uint32_t q0, q1;
-            if ((j & 1) == 0) {  // 18j + 2 + 8(h&1) is 2 mod 4: three dwords, shifted by 2 bytes
-                const uint32_t* p = reinterpret_cast<const uint32_t*>(my_q + 18 * j - 2);
-                const uint32_t w0 = p[0], w1 = p[1], w2 = p[2];
-                q0 = align16(w1, w0);
-                q1 = align16(w2, w1);
-            } else {
-                const uint32_t* p = reinterpret_cast<const uint32_t*>(my_q + 18 * j);
-                q0 = p[0];
-                q1 = p[1];
-            }
-            const uint32_t n0 = (q0 >> nib_shift) & 0x0f0f0f0fu, n1 = (q1 >> nib_shift) & 0x0f0f0f0fu;
-            const long wop = static_cast<long>((static_cast<unsigned long>(n1) << 32) | n0);
-            // f16 scales of rows 16 wv + 4h .. +3
-            const uint2 dwb = *reinterpret_cast<const uint2*>(&s_dw[buf][j * kWgRows + 16 * wv + 4 * h]);
-            const float dw[4] = {h2f(dwb.x & 0xffffu), h2f(dwb.x >> 16), h2f(dwb.y & 0xffffu), h2f(dwb.y >> 16)};
-            long a_nxt[TG];
-            v4i c8_nxt[TG];
-#pragma unroll
-            for (int g = 0; g < TG; ++g) {
-                const v4i is = __builtin_amdgcn_mfma_i32_16x16x32_i8(wop, a_cur[g], c8_cur[g], 0, 0, 0);
-                if (j + 1 < kChunk) {
-                    a_nxt[g] = *reinterpret_cast<const long*>(&s_a[buf][g * 4096 + (j + 1) * 512 + 8 * l]);
-                    c8_nxt[g] = __builtin_amdgcn_mfma_i32_16x16x32_i8(kMinus8, a_nxt[g], v4i{0, 0, 0, 0}, 0, 0, 0);
-                }
-                const float da = s_da[buf][j * kToks + 16 * g + li];
-                acc[g][0] = fmaf(dw[0] * da, static_cast<float>(is[0]), acc[g][0]);
-                acc[g][1] = fmaf(dw[1] * da, static_cast<float>(is[1]), acc[g][1]);
-                acc[g][2] = fmaf(dw[2] * da, static_cast<float>(is[2]), acc[g][2]);
-                acc[g][3] = fmaf(dw[3] * da, static_cast<float>(is[3]), acc[g][3]);
-            }
-            if (j + 1 < kChunk) {
-#pragma unroll
-                for (int g = 0; g < TG; ++g) {
-                    a_cur[g] = a_nxt[g];
-                    c8_cur[g] = c8_nxt[g];
-                }
-            }
-        }
-        store(buf ^ 1);  // the idle buffer was last read in chunk c - 1, before the barrier that ended it
-        __syncthreads();
     }
+    chain(0);
+    chain(1);
 
-    // lane holds (row 16 wv + 4h + v, token 16g + li) of each token group g
+    // lane holds row 32 wr + li, tokens 8 (i / 4) + 4 h + i % 4
+    const int orow = r0 + 32 * wr + li;
+    if (orow < N) {
 #pragma unroll
-    for (int g = 0; g < TG; ++g) {
-        const int tk = t0 + 16 * g + li;
-        if (tk < B) {
-#pragma unroll
-            for (int v = 0; v < 4; ++v) {
-                const int orow = r0 + 16 * wv + 4 * h + v;
-                if (orow < N) y[static_cast<size_t>(tk) * N + orow] = acc[g][v];
-            }
+        for (int i = 0; i < 16; ++i) {
+            const int tk = t0 + 32 * wt + 8 * (i / 4) + 4 * h + i % 4;
+            if (tk < B) y[static_cast<size_t>(tk) * N + orow] = acc[i];
         }
     }
 }
@@ -383,18 +412,25 @@ hipError_t launch_gemm_q4_0_q8_mfma(const uint8_t* W, const int8_t* aq, const fl
         const char* e = getenv("MVH_GEMM_TG2_ROWTILES");
         return e ? static_cast<size_t>(atoll(e)) : static_cast<size_t>(512);
     }();
-    // From 256 tokens the workgroup kernel (64 rows x 32 tokens per workgroup)
-    // is a few percent faster (M = 512: 68-69 against 70-71 us at 4096^2,
-    // 160 against 165-172 us at the other two shapes); at M = 128 it is slower.
-    // Tuning override: MVH_GEMM_WG=0 never, 1 at every batch size.
+    // The workgroup kernel from rows x tokens = 768 K on: below, its 64 x 64
+    // tiles leave CUs idle and a lone wave's chain sets the time (4096x4096 at
+    // 128 tokens 27 against 21 us, 4096->11008 at 64 even at 27.5; 4096x4096 at
+    // 256 29 against 37, 4096->11008 at 128 35 against 42, 4096->22016 at 64 34
+    // against 42).  128-row x 32-token tiles where 64 would leave half of the
+    // last ones empty.  Tuning override: MVH_GEMM_WG=0 never, 1 at every batch
+    // size.
     static const int wg_mode = [] {
         const char* e = getenv("MVH_GEMM_WG");
         return e ? atoi(e) : -1;
     }();
-    const size_t gw = (rows + 63) / 64;
-    if (wg_mode == 1 || (wg_mode != 0 && batch >= 256)) {
-        gemm_q4_0_q8_mfma_wg_kernel<2><<<dim3(static_cast<unsigned>(gw), static_cast<unsigned>(g32)), 256, 0, st>>>(
-            W, aq, ad, y, N, nb, Bn);
+    if (wg_mode == 1 || (wg_mode != 0 && rows * batch >= size_t{768} * 1024)) {
+        if (g32 % 2) {
+            const dim3 grid(static_cast<unsigned>((rows + 127) / 128), static_cast<unsigned>(g32));
+            gemm_q4_0_q8_tile_kernel<1><<<grid, 256, 0, st>>>(W, aq, ad, y, N, nb, Bn);
+        } else {
+            const dim3 grid(static_cast<unsigned>((rows + 63) / 64), static_cast<unsigned>(g32 / 2));
+            gemm_q4_0_q8_tile_kernel<2><<<grid, 256, 0, st>>>(W, aq, ad, y, N, nb, Bn);
+        }
         return hipGetLastError();
     }
     // (17..32 tokens: the row-tile count alone decides -- the fused q|k|v's

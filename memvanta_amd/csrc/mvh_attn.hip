@@ -6,6 +6,8 @@
 // elements: kv_page_bytes), K and V in separate pages -- the PagedKVCache
 // layout of src/llama_model.cpp:18-22.
 #include "mvh_kernels.hpp"
+
+#include <type_traits>
 #define MVH_EXPF_QUAL __device__ __forceinline__
 #define MVH_EXPF_TABLE static __constant__ const
 #include "mvh_expf.h"
@@ -918,9 +920,10 @@ __global__ __launch_bounds__(kSM) void attn_scores_softmax_kernel(const void* co
     }
 }
 
-// Scores of a prefill chunk for F16 pages, K read once per head and row
-// block: workgroup (head h, block of kTR positions), every query token of the
-// chunk (B <= 32).  The block's K rows come in with 16-byte loads (a wave's
+// Scores of a prefill chunk for F16 pages, K read once per head, row block
+// and 32 tokens: workgroup (head h, block of kTR positions, group of up to 32
+// query tokens); a row block past the group's last position has nothing to do.
+// The block's K rows come in with 16-byte loads (a wave's
 // load covers whole rows) into an LDS tile; the chunk's q rows are staged
 // beside it; thread t scores tile row t % kTR for tokens t / kTR + 4k
 // (k = 0..7), with kv_dot_row's order (eight-lane fma over the elements,
@@ -940,7 +943,11 @@ __global__ __launch_bounds__(256) void attn_scores_tile_kernel(const void* const
     __shared__ __align__(16) uint8_t s_kt[kTR * KP];
     __shared__ __align__(16) float s_q[32 * HD];
     const int h = blockIdx.x, r0 = blockIdx.y * kTR, t = threadIdx.x, kh = h / group;
-    const int nmax = pos0 + B;  // rows 0..nmax-1 hold keys (this chunk's included)
+    const int b0 = blockIdx.z * 32;
+    pos0 += b0, B = min(B - b0, 32);
+    q += static_cast<size_t>(b0) * q_pitch, s_out += static_cast<size_t>(b0) * n_head * pitch;
+    const int nmax = pos0 + B;  // rows 0..nmax-1 hold keys (this group's included)
+    if (r0 >= nmax) return;
 #pragma unroll
     for (int i = 0; i < kTR * CPR / 256; ++i) {
         const int pc = i * 256 + t, row = min(r0 + pc / CPR, nmax - 1);
@@ -1029,8 +1036,8 @@ __global__ __launch_bounds__(kSM) void attn_softmax_rows_kernel(float* __restric
 // elements), out[d] = fma(w_t, V_t[d], out[d]) over t = 0..pos0+b in order,
 // as in the reference (w_t the weights attn_scores_softmax_kernel wrote).  V rows come in 64-row tiles staged once in LDS for all
 // 32 tokens (the next tile's loads in flight while a tile is summed); the
-// weights of rows past a token's last position are 0 there, an exact no-op
-// (those rows are the chunk's later tokens, finite).  With q8 the output's
+// rows past a token's last position (the chunk's later tokens, whatever they
+// hold) are left out, lane by lane, in the tiles that have any.  With q8 the output's
 // quantize_q8 blocks (one per token and slice) are written too, row-major or
 // in the prefill GEMM's operand order (q8_op).
 constexpr int kPV = 256;
@@ -1117,7 +1124,6 @@ __global__ __launch_bounds__(kPV) void attn_pv_chunk_kernel(int pos_arg, int B, 
         for (int j = 0; j < 8; ++j) s_at[ar_][ac + j] = areg[j];
         __syncthreads();
         if (r0 + kPVRows < nmax) fetch(r0 + kPVRows);
-        // rows past nmax in the last tile carry weight 0 (areg) over finite rows: no-ops
         const int rows4 = min(kPVRows, (nmax - r0 + 3) & ~3);
         // 4-row steps with two register sets used in turn; every LDS read is
         // unconditional (a step past the last re-reads the last one, unused)
@@ -1131,28 +1137,36 @@ __global__ __launch_bounds__(kPV) void attn_pv_chunk_kernel(int pos_arg, int B, 
 #pragma unroll
             for (int i = 0; i < 4; ++i) v[i] = *reinterpret_cast<const R*>(&s_v[r + i][dq]);
         };
-        auto step = [&](float (&c)[4], const float4& w4, const R (&v)[4]) {
-            const float w[4] = {w4.x, w4.y, w4.z, w4.w};
+        auto sum_tile = [&](auto masked) __attribute__((always_inline)) {
+            auto step = [&](float (&c)[4], int st, const float4& w4, const R (&v)[4]) {
+                const float w[4] = {w4.x, w4.y, w4.z, w4.w};
 #pragma unroll
-            for (int i = 0; i < 4; ++i)
+                for (int i = 0; i < 4; ++i)
 #pragma unroll
-                for (int k = 0; k < 4; ++k) c[k] = fmaf(w[i], PvRaw<KT>::at(v[i], k), c[k]);
+                    for (int k = 0; k < 4; ++k) {
+                        const float s = fmaf(w[i], PvRaw<KT>::at(v[i], k), c[k]);
+                        c[k] = !decltype(masked)::value || r0 + 4 * st + i < nb ? s : c[k];
+                    }
+            };
+            float4 wa, wb;
+            R va[4], vb[4];
+            ld(0, wa, va);
+            for (int st = 0; st < nst; st += 2) {
+                ld(st + 1, wb, vb);
+                __builtin_amdgcn_sched_barrier(0);
+                step(acc, st, wa, va);
+                __builtin_amdgcn_sched_barrier(0);
+                ld(st + 2, wa, va);
+                __builtin_amdgcn_sched_barrier(0);
+                float nx[4] = {acc[0], acc[1], acc[2], acc[3]};  // the odd step, kept when it exists
+                step(nx, st + 1, wb, vb);
+#pragma unroll
+                for (int k = 0; k < 4; ++k) acc[k] = st + 1 < nst ? nx[k] : acc[k];
+            }
         };
-        float4 wa, wb;
-        R va[4], vb[4];
-        ld(0, wa, va);
-        for (int st = 0; st < nst; st += 2) {
-            ld(st + 1, wb, vb);
-            __builtin_amdgcn_sched_barrier(0);
-            step(acc, wa, va);
-            __builtin_amdgcn_sched_barrier(0);
-            ld(st + 2, wa, va);
-            __builtin_amdgcn_sched_barrier(0);
-            float nx[4] = {acc[0], acc[1], acc[2], acc[3]};  // the odd step, kept when it exists
-            step(nx, wb, vb);
-#pragma unroll
-            for (int k = 0; k < 4; ++k) acc[k] = st + 1 < nst ? nx[k] : acc[k];
-        }
+        // a tile with rows that some of the 32 tokens do not see, or one without
+        if (r0 + kPVRows > pos0 + b0 + 1) sum_tile(std::true_type{});
+        else sum_tile(std::false_type{});
         __syncthreads();
     }
     if (b >= B) return;  // whole 8-lane groups (one token) leave together
@@ -1238,10 +1252,11 @@ hipError_t attn_prefill_typed(const void* const* pt_k, const void* const* pt_v, 
                               size_t kv_dim, size_t page_tokens, hipStream_t st) {
     const int group = static_cast<int>(n_head / n_head_kv);
     const int pitch = static_cast<int>(max_pos);  // weight row pitch >= last position + 1
-    if (kScoresTile && KT == kKvF16 && !d_pos && B >= 8 && B <= 32 && (hd == 128 || hd == 64) && q_pitch % 4 == 0 &&
+    if (kScoresTile && KT == kKvF16 && !d_pos && B >= 8 && (hd == 128 || hd == 64) && q_pitch % 4 == 0 &&
         (reinterpret_cast<uintptr_t>(q) & 15) == 0) {
-        // F16 chunks of 8..32 tokens, q rows 16-byte aligned: K staged once per (head, 64-row block)
-        const dim3 gs(static_cast<unsigned>(n_head), static_cast<unsigned>((pos + B + kTR - 1) / kTR));
+        // F16 chunks of 8 tokens or more, q rows 16-byte aligned: K staged once per (head, 64-row block, 32 tokens)
+        const dim3 gs(static_cast<unsigned>(n_head), static_cast<unsigned>((pos + B + kTR - 1) / kTR),
+                      static_cast<unsigned>((B + 31) / 32));
         if (hd == 128)
             attn_scores_tile_kernel<128><<<gs, 256, 0, st>>>(pt_k, q, static_cast<int>(q_pitch), a_scratch,
                                                              static_cast<int>(pos), static_cast<int>(B),

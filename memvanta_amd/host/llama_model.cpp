@@ -161,7 +161,8 @@ LlamaModel::LlamaModel(const std::string& path, int device, std::size_t ctx_over
     check(hipMemcpy(pt_k_, tk.data(), tk.size() * sizeof(void*), hipMemcpyHostToDevice), "page table");
     check(hipMemcpy(pt_v_, tv.data(), tv.size() * sizeof(void*), hipMemcpyHostToDevice), "page table");
 
-    const std::size_t B = max_batch_, D = c_.n_embd, F = c_.n_ff, KV = c_.kv_dim(), W = std::max(D, F);
+    step_tokens_ = std::max(max_batch_, std::min<std::size_t>(kStepTokens, c_.n_ctx));
+    const std::size_t B = step_tokens_, D = c_.n_embd, F = c_.n_ff, KV = c_.kv_dim(), W = std::max(D, F);
     for (Lane& l : lanes_) {
         if (&l != &lanes_[0]) check(hipStreamCreateWithFlags(&l.st, hipStreamNonBlocking), "hipStreamCreate");
         l.x = static_cast<float*>(dalloc(B * D * 4));
@@ -623,6 +624,24 @@ const std::vector<float>& LlamaModel::forward(int token, bool compute_logits) {
     return logits_;
 }
 
+const char* LlamaModel::chunk_error(const std::vector<int>& tokens, std::size_t i, std::size_t B) const {
+    if (pos_ + B > c_.n_ctx) return "context exhausted";
+    for (std::size_t b = i; b < i + B; ++b)
+        if (tokens[b] < 0 || static_cast<std::size_t>(tokens[b]) >= c_.vocab) return "token id out of range";
+    return nullptr;
+}
+
+// Whether consecutive chunks of `batch` tokens (and a last one of 2 or more)
+// give the same bits in one step.  A token's results depend on its chunk only
+// through the arithmetic the chunk's size selects for it: in the fp32
+// numerics the last B % 8 (feed-forward) or B % 4 tokens of a chunk take the
+// per-token dots, so whole multiples of 8 join, and the last chunk's leftover
+// tokens are the joined step's; in the Q8 numerics every token of a chunk of
+// 2 or more is treated alike (one of 1 has its own path).
+bool LlamaModel::chunks_join(std::size_t batch) const {
+    return mode_ == PrefillMode::Q8 ? batch >= 2 : batch % 8 == 0;
+}
+
 const std::vector<float>& LlamaModel::prefill(const std::vector<int>& tokens, std::size_t batch_size,
                                               bool compute_logits_last) {
     if (tokens.empty()) return logits_;
@@ -649,14 +668,17 @@ const std::vector<float>& LlamaModel::prefill(const std::vector<int>& tokens, st
         if (!quiet) check(first, "sync");
     };
     try {
-        for (std::size_t i = 0; i < tokens.size(); i += batch_size, ++chunk) {
-            const std::size_t B = std::min(batch_size, tokens.size() - i);
-            const char* err = nullptr;
-            if (pos_ + B > c_.n_ctx) err = "context exhausted";
-            for (std::size_t b = 0; b < B && !err; ++b)
-                if (tokens[i + b] < 0 || static_cast<std::size_t>(tokens[i + b]) >= c_.vocab)
-                    err = "token id out of range";
-            if (err) throw std::runtime_error(err);  // the chunks before this one complete (drained below)
+        std::size_t B = 0;
+        for (std::size_t i = 0; i < tokens.size(); i += B, ++chunk) {
+            B = std::min(batch_size, tokens.size() - i);
+            // the chunks before a refused one complete (drained below)
+            if (const char* err = chunk_error(tokens, i, B)) throw std::runtime_error(err);
+            // later chunks join the step while that leaves every result as it is
+            while (!profiling_ && i + B < tokens.size() && chunks_join(batch_size)) {
+                const std::size_t next = std::min(batch_size, tokens.size() - i - B);
+                if (next < 2 || B + next > step_tokens_ || chunk_error(tokens, i, B + next)) break;
+                B += next;
+            }
             const bool last = compute_logits_last && i + B == tokens.size();
             const int lane = static_cast<int>(chunk % lanes);
             ln_ = &lanes_[lane];

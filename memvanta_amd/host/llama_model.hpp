@@ -90,15 +90,18 @@ private:
     void decode_step(const int* d_token, bool logits, bool argmax);
     void store_kv(const QkvLayout& lay, void* const* pk, void* const* pv, const int* d_pos, std::size_t pos,
                   std::size_t B);
-    // one prefill chunk on lane ln_; prev_lane >= 0: the previous chunk runs on
-    // that lane and this chunk's attention of layer l waits for its KV of layer l
+    const char* chunk_error(const std::vector<int>& tokens, std::size_t i, std::size_t B) const;
+    bool chunks_join(std::size_t batch) const;
+    // one prefill step (a chunk, or consecutive ones joined) on lane ln_;
+    // prev_lane >= 0: the previous step runs on that lane and this step's
+    // attention of layer l waits for its KV of layer l
     void batch_step(const int* tokens, std::size_t B, bool logits, int prev_lane = -1);
     void check(hipError_t e, const char* what) const;
 
     // A lane: a stream and the activation buffers of one step in flight
-    // ([max_batch][...] for prefill; row 0 for decode).  Decode runs on lane 0;
-    // consecutive prefill chunks take the lanes in turn, so chunk c + 1
-    // computes layer l while chunk c computes layer l + 1.
+    // ([step_tokens_][...] for prefill; row 0 for decode).  Decode runs on lane
+    // 0; consecutive prefill steps take the lanes in turn, so step c + 1
+    // computes layer l while step c computes layer l + 1.
     struct Lane {
         hipStream_t st{};
         float *x{}, *n{}, *qkv{}, *att{}, *proj{}, *gu{}, *ff{}, *scores{};
@@ -114,12 +117,17 @@ private:
     // three lanes: pp512 of the 7B shape 7.55 K (one) / 10.3 K (two) / 11.1 K
     // (three) / 10.1 K (four) tok/s; GPU_MAX_HW_QUEUES is 4
     static constexpr int kLanes = 3;
+    // Tokens that joined chunks may fill: one launch of every kernel then does
+    // the work of 256 / batch chunks.  512 tokens in chunks of 32, as they are /
+    // joined to 128 / 256 / 512 tokens: 7B shape, 4 layers, Q8 5.35 / 3.25 /
+    // 2.51 / 2.56 ms; TinyLlama shape, 8 layers, fp32 8.33 / 6.91 / 6.47 / 6.80.
+    static constexpr std::size_t kStepTokens = 256;
     Lane lanes_[kLanes];
     Lane* ln_{&lanes_[0]};             // the lane the step helpers launch on
     std::vector<hipEvent_t> kv_done_;  // [lane][layer]: the KV rows of the lane's chunk at that layer are written
     int kv_type_{1};
     PrefillMode mode_;
-    std::size_t page_tokens_{}, max_pages_{}, max_batch_{}, pos_{}, kv_hi_{};
+    std::size_t page_tokens_{}, max_pages_{}, max_batch_{}, step_tokens_{}, pos_{}, kv_hi_{};
     Tensor embd_, out_;
     float* out_norm_{};
     std::vector<Layer> layers_;

@@ -1,0 +1,74 @@
+"""Prefill chunks joined into one step, and what a joined step must not change: the state a refused chunk leaves
+behind, and the independence of a token from the rows of later ones."""
+import dataclasses
+
+import numpy as np
+import pytest
+
+from memvanta_amd import capi, synth
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(scope="module")
+def tiny(tmp_path_factory):
+    path = str(tmp_path_factory.mktemp("joined") / "tiny.gguf")
+    synth.write_model(dataclasses.replace(synth.TINY, ctx=384), path, seed=1234)
+    return path
+
+
+@pytest.mark.parametrize("mode", [0, 1])
+@pytest.mark.parametrize("bad,batch,done", [(45, 8, 40), (0, 16, 0), (79, 16, 64), (33, 32, 32)])
+def test_refused_chunk_leaves_the_earlier_ones(tiny, mode, bad, batch, done):
+    """The chunks before the one with a bad token complete, whichever steps they were joined into."""
+    prompt = synth.prompt_tokens(3, 80).astype(np.int32)
+    m = capi.Model(tiny, ctx=256, act_mode=mode, max_batch=32)
+    broken = prompt.copy()
+    broken[bad] = 32000
+    with pytest.raises(capi.MvhError, match="token id out of range"):
+        m.prefill(broken, batch)
+    assert m.position == done
+    got = m.prefill(prompt[done:], batch).copy()
+    m.reset()
+    assert (got.view(np.uint32) == m.prefill(prompt, batch).view(np.uint32)).all()
+    m.close()
+
+
+def test_context_end_inside_a_step(tiny):
+    m = capi.Model(tiny, ctx=50, max_batch=16)
+    with pytest.raises(capi.MvhError, match="context exhausted"):
+        m.prefill(synth.prompt_tokens(3, 60).astype(np.int32), 16)
+    assert m.position == 48
+    m.close()
+
+
+@pytest.mark.parametrize("mode,n,batch", [(0, 100, 8), (0, 77, 24), (0, 70, 4), (1, 99, 7), (1, 65, 32), (1, 259, 64)])
+def test_joined_equals_single_chunks(tiny, mode, n, batch):
+    """Steps at and over their 256 tokens, ragged last chunks of 1, 2 and more, and batches that do not join."""
+    prompt = synth.prompt_tokens(5, n).astype(np.int32)
+    m = capi.Model(tiny, ctx=320, act_mode=mode, max_batch=64)
+    got = m.prefill(prompt, batch).copy()
+    m.reset()
+    for i in range(0, n, batch):
+        want = m.prefill(prompt[i:i + batch], batch)
+    assert (got.view(np.uint32) == want.view(np.uint32)).all()
+    m.close()
+
+
+@pytest.mark.parametrize("kv_type", [capi.MVH_KV_F32, capi.MVH_KV_F16])
+@pytest.mark.parametrize("B", [31, 40])
+def test_later_rows_do_not_reach_earlier_tokens(ctx, kv_type, B):
+    """V rows past a token's position may hold anything: an infinity there leaves the token's output as it was."""
+    rng = np.random.default_rng(B)
+    n_head, hd, pos = 4, 64, 70
+    k, v = (rng.standard_normal((pos + B, n_head * hd), dtype=np.float32) for _ in range(2))
+    q = rng.standard_normal((B, n_head * hd), dtype=np.float32)
+    outs = []
+    for far in (0.5, np.inf):
+        v[pos + B - 3:] = far
+        kv = ctx.kv_cache(1, n_head * hd, 16, 256, kv_type=kv_type)
+        kv.write(0, 0, k, v)
+        outs.append(kv.attn_batch(0, q, pos, B, n_head, n_head, hd).copy())
+        kv.close()
+    a, b = (o[: B - 3].view(np.uint32) for o in outs)
+    assert (a == b).all()

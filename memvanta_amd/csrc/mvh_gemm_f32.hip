@@ -14,9 +14,8 @@
 //       (src/gguf_kernels.cpp:191-216): t_e runs over all blocks without
 //       reset, term = fma(float(q)*d, x, t_e) with float(q)*d rounded first,
 //       result t0+t1+..+t7;
-//   batch_blocksum_kernel  dot_q4_0_fp32 / dot_q8_0_fp32 (:93-120) and the
-//       native dot_q4_0 / dot_q8_0 (src/quant.cpp:87-156): per block t_e from
-//       zero, s = 0+t0+..+t7, then sum = fma(d, s, sum) over the blocks.
+//   batch_blocksum_kernel  dot_q4_0_fp32 / dot_q8_0_fp32 (:93-120): per block
+//       t_e from zero, s = 0+t0+..+t7, then sum = fma(d, s, sum) over the blocks.
 #include "mvh_kernels.hpp"
 
 #include <cstdlib>
@@ -27,32 +26,17 @@ namespace {
 
 typedef float v4f __attribute__((ext_vector_type(4)));
 
-// Block geometry of a weight type: bytes, first quant byte, 16-byte pieces of
-// an 8-block unit.
+// Bytes of a block: a 2-byte scale, then the quants.
 template <uint32_t TYPE>
 struct Fmt;
 template <>
 struct Fmt<kQ4_0> {
-    static constexpr int kB = 18, kQ = 2;
+    static constexpr int kB = 18;
 };
 template <>
 struct Fmt<kQ8_0> {
-    static constexpr int kB = 34, kQ = 2;
+    static constexpr int kB = 34;
 };
-template <>
-struct Fmt<kNQ4_0> {
-    static constexpr int kB = 20, kQ = 4;
-};
-template <>
-struct Fmt<kNQ8_0> {
-    static constexpr int kB = 36, kQ = 4;
-};
-
-template <uint32_t TYPE>
-__device__ __forceinline__ float block_scale(const uint8_t* blk) {
-    if constexpr (Fmt<TYPE>::kQ == 2) return h2f(*reinterpret_cast<const uint16_t*>(blk));
-    else return *reinterpret_cast<const float*>(blk);
-}
 
 // The four weights of one operand dword, times the block's scale.  Q4_0 (v: four
 // codes q, one per byte's low nibble, bit 3 flipped, so a nibble is q - 8 in
@@ -385,6 +369,141 @@ hipError_t launch_chain(const uint8_t* W, const float* x, float* y, size_t rows,
     return hipGetLastError();
 }
 
+// ---- per-block sums (the per-token fp32 dots over several tokens) --------------
+//
+// A workgroup owns 16*R rows x 16 tokens.  The block sums are independent of
+// each other, so its four waves take them in turn, four blocks (a step) each;
+// the sums and the scales meet in LDS, and per round of 16 blocks every thread
+// runs the in-order fma chain of its R outputs over them.  A wave's weight
+// bytes of a step pass through an LDS copy of its own; the activations are the
+// other operand as they lie in memory (8 floats per lane and block).  Both are
+// fetched one round ahead.
+// What bounds it: eight f32 MFMAs (256 cycles) and the 28 adds of their lane
+// sums per 16 x 16 outputs and block, which exclude each other; with a
+// workgroup or less per CU, the latency of a round (about 2 us).
+// Against the VALU kernels before (us): Q8_0 2048->5632 at 5 / 16 / 64 / 256
+// tokens 22.6 / 25.2 / 51.9 / 161 -> 13.0 / 15.7 / 30.8 / 96; Q4_0 4096->11008
+// 55 / 58 / 167 / 604 -> 28.5 / 33.1 / 102 / 346.
+template <uint32_t TYPE, int R>
+__global__ __launch_bounds__(kT) void batch_blocksum_kernel(const uint8_t* __restrict__ W, const float* __restrict__ x,
+                                                            float* __restrict__ y, int N, int nb, int B) {
+    constexpr int kS = 4, kRound = 4 * kS;        // blocks per step, per round
+    constexpr int kB = Fmt<TYPE>::kB, kUB = kS * kB, kPitch = kUB + 4;  // an odd number of dwords
+    constexpr int kRows = 16 * R, kPieces = kRows * (kUB / 8), kN = (kPieces + 63) / 64;
+    static_assert(kUB % 8 == 0);
+    __shared__ __align__(16) uint8_t s_w[4][kRows * kPitch + 8];  // + a spare slot for unused stores
+    __shared__ float s_s[kRound][R][4][64];                       // [block][row group][token v of lane][lane]
+    __shared__ float s_d[kRound][kRows];
+    const int t = threadIdx.x, l = t & 63, w = __builtin_amdgcn_readfirstlane(t >> 6), li = l & 15, m = l >> 4;
+    const int row0 = blockIdx.x * kRows, tok0 = blockIdx.y * 16;
+    const int steps = nb / kS, K = nb * 32, row_bytes = nb * kB;
+
+    const uint8_t* wbase = W + static_cast<size_t>(row0) * row_bytes;
+    uint32_t src[kN];
+    int dst[kN];
+#pragma unroll
+    for (int i = 0; i < kN; ++i) {
+        const int p = l + 64 * i, pc = min(p, kPieces - 1), row = pc / (kUB / 8), k = pc % (kUB / 8);
+        // rows past N read row N - 1, tokens past B token B - 1 (not stored)
+        src[i] = static_cast<uint32_t>(min(row, N - 1 - row0)) * static_cast<uint32_t>(row_bytes) + 8 * k;
+        dst[i] = p < kPieces ? row * kPitch + 8 * k : kRows * kPitch;
+    }
+    const float* xbase = x + static_cast<size_t>(tok0) * K;
+    const uint32_t xoff = 4u * (static_cast<uint32_t>(min(li, B - 1 - tok0)) * static_cast<uint32_t>(K) + 8 * m);
+    uint2 wreg[kN];
+    float4 xreg[kS][2];
+    auto load = [&](int step) __attribute__((always_inline)) {
+        const uint8_t* p = wbase + step * kUB;
+#pragma unroll
+        for (int i = 0; i < kN; ++i) wreg[i] = ld_at<uint2>(p, src[i]);
+#pragma unroll
+        for (int j = 0; j < kS; ++j) {
+            xreg[j][0] = ld_at<float4>(xbase + (step * kS + j) * 32, xoff);
+            xreg[j][1] = ld_at<float4>(xbase + (step * kS + j) * 32 + 4, xoff);
+        }
+    };
+    // the lane's operand bytes of a block: Q4_0 elements 8m .. are nibbles m >> 1 of bytes 8 (m & 1) ..
+    const int rowo = li * kPitch, qo = rowo + (TYPE == kQ4_0 ? 8 * (m & 1) : 8 * m);
+    const int nib_sh = 4 * (m >> 1);
+    float sum[R];
+#pragma unroll
+    for (int r = 0; r < R; ++r) sum[r] = 0.f;
+
+    load(min(w, steps - 1));
+    for (int r0 = 0; r0 < steps; r0 += 4) {
+        float4 xc[kS][2];
+#pragma unroll
+        for (int j = 0; j < kS; ++j) xc[j][0] = xreg[j][0], xc[j][1] = xreg[j][1];
+#pragma unroll
+        for (int i = 0; i < kN; ++i) {
+            uint32_t* p = reinterpret_cast<uint32_t*>(s_w[w] + dst[i]);
+            p[0] = wreg[i].x, p[1] = wreg[i].y;
+        }
+        load(min(r0 + 4 + w, steps - 1));
+        __builtin_amdgcn_wave_barrier();
+        if (r0 + w < steps) {
+#pragma unroll
+            for (int j = 0; j < kS; ++j) {
+                const float xv[8] = {xc[j][0].x, xc[j][0].y, xc[j][0].z, xc[j][0].w,
+                                     xc[j][1].x, xc[j][1].y, xc[j][1].z, xc[j][1].w};
+#pragma unroll
+                for (int r = 0; r < R; ++r) {
+                    const uint8_t* wr = s_w[w] + r * 16 * kPitch + j * kB;
+                    uint32_t q[2];
+                    if ((j * kB) & 2) {  // the quants are dword aligned
+                        const uint32_t* p = reinterpret_cast<const uint32_t*>(wr + qo + 2);
+                        q[0] = p[0], q[1] = p[1];
+                    } else {
+                        const uint32_t* p = reinterpret_cast<const uint32_t*>(wr + qo);
+                        q[0] = align16(p[1], p[0]), q[1] = align16(p[2], p[1]);
+                    }
+                    if (m == 0)
+                        s_d[w * kS + j][16 * r + li] = h2f(*reinterpret_cast<const uint16_t*>(wr + rowo));
+                    float a[2][4];
+#pragma unroll
+                    for (int e = 0; e < 2; ++e) {
+                        if constexpr (TYPE == kQ4_0)
+                            weights<TYPE, 4>((q[e] ^ 0x88888888u) >> nib_sh, 16.0f, a[e]);
+                        else
+                            weights<TYPE, 4>(q[e], 1.0f, a[e]);
+                    }
+                    v4f te[8];
+#pragma unroll
+                    for (int e = 0; e < 8; ++e)
+                        te[e] = __builtin_amdgcn_mfma_f32_16x16x4f32(xv[e], a[e >> 2][e & 3], v4f{0.f, 0.f, 0.f, 0.f}, 0, 0, 0);
+                    v4f s = te[0];
+#pragma unroll
+                    for (int e = 1; e < 8; ++e)
+#pragma unroll
+                        for (int v = 0; v < 4; ++v) s[v] = s[v] + te[e][v];
+#pragma unroll
+                    for (int v = 0; v < 4; ++v) s_s[w * kS + j][r][v][l] = s[v];
+                }
+            }
+        }
+        __syncthreads();
+        for (int b0 = 0; b0 < min(kRound, nb - r0 * kS); b0 += 8)  // whole halves of a round: nb % 8 == 0
+#pragma unroll
+            for (int b = 0; b < 8; ++b)
+#pragma unroll
+                for (int r = 0; r < R; ++r) sum[r] = fmaf(s_d[b0 + b][16 * r + li], s_s[b0 + b][r][w][l], sum[r]);
+        __syncthreads();
+    }
+    // wave w, lane l: token 4m + w, row li of each row group
+    const int tk = tok0 + 4 * m + w;
+#pragma unroll
+    for (int r = 0; r < R; ++r) {
+        const int row = row0 + 16 * r + li;
+        if (row < N && tk < B) y[static_cast<size_t>(tk) * N + row] = sum[r];
+    }
+}
+
+template <uint32_t TYPE, int R>
+void blocksum_one(const uint8_t* W, const float* x, float* y, int N, int nb, int B, hipStream_t st) {
+    const dim3 grid(static_cast<unsigned>((N + 16 * R - 1) / (16 * R)), static_cast<unsigned>((B + 15) / 16));
+    batch_blocksum_kernel<TYPE, R><<<grid, kT, 0, st>>>(W, x, y, N, nb, B);
+}
+
 }  // namespace
 
 hipError_t launch_batch4_f32act(uint32_t type, const uint8_t* W, const float* x, float* y, size_t rows, size_t cols,
@@ -392,6 +511,29 @@ hipError_t launch_batch4_f32act(uint32_t type, const uint8_t* W, const float* x,
     if (!rows || !batch) return hipSuccess;
     return type == kQ4_0 ? launch_chain<kQ4_0>(W, x, y, rows, cols, batch, st)
                          : launch_chain<kQ8_0>(W, x, y, rows, cols, batch, st);
+}
+
+bool batch_blocksum_ok(uint32_t type, const uint8_t* W, size_t cols) {
+    return (type == kQ4_0 || type == kQ8_0) && cols % 256 == 0 && (reinterpret_cast<uintptr_t>(W) & 15) == 0;
+}
+
+hipError_t launch_batch_blocksum(uint32_t type, const uint8_t* W, const float* x, float* y, size_t rows, size_t cols,
+                                 size_t batch, hipStream_t st) {
+    if (!rows || !batch) return hipSuccess;
+    if (!batch_blocksum_ok(type, W, cols)) return hipErrorInvalidValue;
+    const int N = static_cast<int>(rows), nb = static_cast<int>(cols / 32), B = static_cast<int>(batch);
+    // 32-row tiles read the activations half as often; 16-row ones where those
+    // would be fewer than two workgroups per CU (2048->5632 Q8_0 at 32 / 64
+    // tokens: 16 rows 19.9 / 35.9 us, 32 rows 23.4 / 30.8)
+    const int R = (rows + 31) / 32 * ((batch + 15) / 16) >= 512 ? 2 : 1;
+    if (type == kQ4_0) {
+        if (R == 2) blocksum_one<kQ4_0, 2>(W, x, y, N, nb, B, st);
+        else blocksum_one<kQ4_0, 1>(W, x, y, N, nb, B, st);
+    } else {
+        if (R == 2) blocksum_one<kQ8_0, 2>(W, x, y, N, nb, B, st);
+        else blocksum_one<kQ8_0, 1>(W, x, y, N, nb, B, st);
+    }
+    return hipGetLastError();
 }
 
 }  // namespace mvh

@@ -72,6 +72,11 @@ hipError_t launch_gemv_q4_0_f32act(const uint8_t* W, const float* x, float* y, s
 // q4/q8_row_batch4_fp32 numerics per (row, token) for Q4_0 / Q8_0
 hipError_t launch_batch4_f32act(uint32_t type, const uint8_t* W, const float* x, float* y, size_t rows, size_t cols,
                                 size_t batch, hipStream_t st);
+// The per-token fp32 dots (dot_q4_0_fp32 / dot_q8_0_fp32) of a whole batch on
+// the f32 matrix pipe: Q4_0 / Q8_0, cols % 256 == 0, W 16-byte aligned.
+bool batch_blocksum_ok(uint32_t type, const uint8_t* W, size_t cols);
+hipError_t launch_batch_blocksum(uint32_t type, const uint8_t* W, const float* x, float* y, size_t rows, size_t cols,
+                                 size_t batch, hipStream_t st);
 
 // ---- batched prefill on int8 MFMA (mvh_gemm_q4.hip) ----
 // y[b*rows + r] = dot_q4_q8(W row r, Q8 activation row b) for b < batch

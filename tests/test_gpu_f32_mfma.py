@@ -29,3 +29,19 @@ def test_chain_tiles_bitexact(ctx, oracle, ty, batch, k, n):
     got = ctx.matmul_batch_v06(t, x, capi.MVH_ACT_REF)
     assert_bitexact(got, oracle.matmul_batch_v06(w, ty, n, k, x, is_ffn=False, force_q8=False), f"B={batch} K={k} N={n}")
     t.free()
+
+
+# tokens: the first batch on this kernel, one short of and past its 16-token tiles; rows at the edges of 16 and 32, on
+# both sides of the 512-workgroup line; K: half a round of 16 blocks, one, one and a half, many
+@pytest.mark.parametrize("ty", [synth.Q4_0, synth.Q8_0])
+@pytest.mark.parametrize("batch,k,n", [(4, 256, 1), (5, 512, 17), (15, 768, 31), (16, 1024, 33), (17, 4096, 100),
+                                       (7, 4352, 4096), (64, 256, 4097), (250, 512, 1025), (33, 1280, 5600)])
+def test_block_sums_bitexact(ctx, oracle, ty, batch, k, n):
+    rng = np.random.default_rng(batch * 5 + k + n + ty)
+    w, x = _case(rng, ty, n, k, batch)
+    t = ctx.upload("blk.0.attn_q.weight", ty, k, n, w)
+    want = oracle.matmul_batch(w, ty, n, k, x)
+    assert_bitexact(ctx.matmul_batch(t, x), want, f"B={batch} K={k} N={n}")
+    if ty == synth.Q8_0:
+        assert_bitexact(ctx.matmul_batch_v06(t, x, capi.MVH_ACT_Q8), want, f"v06 q8 B={batch} K={k} N={n}")
+    t.free()

@@ -1190,6 +1190,280 @@ __global__ __launch_bounds__(kPV) void attn_pv_chunk_kernel(int pos_arg, int B, 
     }
 }
 
+// ---- one token over a long cache (C ABI decode attention, hd % 32 == 0) ----------
+//
+// Scores over workgroups of 64 positions, then softmax and the value chains
+// per (head, 32-element slice).
+
+// Raw score of head h (grid x) at position 64 * blockIdx.y + thread: the row's
+// pieces all requested before the first fma (HD 64 / 128; HD = 0: any hd).
+template <int KT, int HD>
+__global__ __launch_bounds__(64) void attn_decode_scores_kernel(const void* const* __restrict__ pt_k,
+                                                                const float* __restrict__ q,
+                                                                float* __restrict__ scores, int n, int group, int hd,
+                                                                int kv_dim, int page_tokens) {
+    extern __shared__ __align__(16) float s_q[];
+    const int h = blockIdx.x, kh = h / group, p = static_cast<int>(blockIdx.y) * 64 + static_cast<int>(threadIdx.x);
+    const int r = min(p, n - 1);
+    const void* page = pt_k[r / page_tokens];
+    const void* row = kv_elem_ptr<KT>(page, r % page_tokens, kv_dim, kh * hd);
+    float sum;
+    if constexpr (HD > 0) {
+        KvRaw8<KT> k[HD / 8];
+#pragma unroll
+        for (int c = 0; c < HD / 8; ++c) k[c] = kv_raw8<KT>(row, 8 * c);
+        for (int i = threadIdx.x; i < HD; i += 64) s_q[i] = q[static_cast<size_t>(h) * HD + i];
+        __syncthreads();
+        float acc[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int c = 0; c < HD / 8; ++c) {  // kv_dot_row's order
+            float kf[8];
+            kv_cvt8<KT>(k[c], kf);
+#pragma unroll
+            for (int e = 0; e < 8; ++e) acc[e] = fmaf(s_q[8 * c + e], kf[e], acc[e]);
+        }
+        sum = acc[0];
+#pragma unroll
+        for (int e = 1; e < 8; ++e) sum = sum + acc[e];
+    } else {
+        for (int i = threadIdx.x; i < hd; i += 64) s_q[i] = q[static_cast<size_t>(h) * hd + i];
+        __syncthreads();
+        sum = kv_dot_row<KT>(row, s_q, hd);
+    }
+    if constexpr (KT == kKvQ8) sum = sum * kv_row_scale<KT>(page, r % page_tokens, page_tokens, kv_dim);
+    if (p < n) scores[static_cast<size_t>(h) * n + p] = __fdiv_rn(sum, sqrt_rn(static_cast<float>(hd)));
+}
+
+// Four consecutive rows of one element, as the value chain reads them.
+template <int KT>
+struct Rows4;
+template <>
+struct Rows4<kKvF32> {
+    typedef float4 T;
+    static __device__ __forceinline__ float at(const T& v, int i) { return i == 0 ? v.x : i == 1 ? v.y : i == 2 ? v.z : v.w; }
+    static __device__ __forceinline__ T pack(const KvRaw8<kKvF32> (&r)[4], int e) {
+        float f[4];
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            const uint4 h = e < 4 ? r[i].a : r[i].b;
+            f[i] = __uint_as_float((e & 3) == 0 ? h.x : (e & 3) == 1 ? h.y : (e & 3) == 2 ? h.z : h.w);
+        }
+        return make_float4(f[0], f[1], f[2], f[3]);
+    }
+};
+template <>
+struct Rows4<kKvF16> {
+    typedef half4v T;
+    static __device__ __forceinline__ float at(const T& v, int i) { return static_cast<float>(v[i]); }
+    static __device__ __forceinline__ T pack(const KvRaw8<kKvF16> (&r)[4], int e) {
+        T v;
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            const uint32_t w = e < 2 ? r[i].a.x : e < 4 ? r[i].a.y : e < 6 ? r[i].a.z : r[i].a.w;
+            v[i] = __builtin_bit_cast(_Float16, static_cast<uint16_t>(w >> (16 * (e & 1))));
+        }
+        return v;
+    }
+};
+template <>
+struct Rows4<kKvQ8> {
+    typedef uint32_t T;
+    static __device__ __forceinline__ float at(const T& v, int i) {
+        return static_cast<float>(static_cast<int8_t>(v >> (8 * i)));
+    }
+    static __device__ __forceinline__ T pack(const KvRaw8<kKvQ8> (&r)[4], int e) {
+        T v = 0;
+#pragma unroll
+        for (int i = 0; i < 4; ++i) v |= ((e < 4 ? r[i].a.x : r[i].a.y) >> (8 * (e & 3)) & 0xffu) << (8 * i);
+        return v;
+    }
+};
+
+// Softmax of a head's raw scores and its value chains over 32 elements of the
+// head (grid y), out[d] = fma(w_t, V_t[d], out[d]) over t in order.  The chain
+// is serial: one wave runs it (a lane per element) while four others first
+// compute the softmax (attn_softmax_rows_kernel's arithmetic and thread
+// mapping) and then stage V ahead of it in tiles, transposed to four rows of
+// an element, so that the chain takes one LDS read of V and one of the weights
+// per four rows.
+// What bounds it: the chain, about 17 cycles a row (more V in flight, three
+// tiles instead of one, changes nothing).  Against one workgroup per head for
+// scores and softmax and 8 chain lanes per 256-thread workgroup, with the
+// position's own write, one call after another (us): 32 heads of 128, F16, at
+// position 600 / 1500 / 3999 29 / 58 / 151 -> 14 / 20 / 41; Q8 33 / 68 / 177 ->
+// 16 / 24 / 50; F32 34 / 72 / 180 -> 16 / 28 / 59.
+constexpr int kDvThreads = 64 + kSM;
+template <int KT>
+struct DvTile {
+    typedef typename Rows4<KT>::T T;
+    static constexpr int kRows = KT == kKvF32 ? 128 : 256;  // rows of a tile
+    static constexpr int kQuads = kRows / 4;
+    static constexpr int kPitch = 32 * sizeof(T) + (KT == kKvF32 ? 16 : sizeof(T));  // bytes of a quad, padded
+    static constexpr int kBytes = kQuads * kPitch;
+};
+template <int KT>
+__global__ __launch_bounds__(kDvThreads) void attn_decode_v_kernel(const void* const* __restrict__ pt_v,
+                                                                   const float* __restrict__ scores,
+                                                                   float* __restrict__ out, int n, int group, int hd,
+                                                                   int kv_dim, int page_tokens) {
+    typedef typename Rows4<KT>::T T;
+    using Tile = DvTile<KT>;
+    extern __shared__ __align__(16) float s_a[];  // [n rounded up to 4] weights
+    __shared__ __align__(16) uint8_t s_v[2][Tile::kBytes];
+    __shared__ float red_f[kSM / 64];
+    __shared__ double red_d[kSM / 64];
+    __shared__ uint64_t s_tab[32];
+    const int h = blockIdx.x, slice = blockIdx.y, kh = h / group;
+    const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int t = static_cast<int>(threadIdx.x) - 64;  // softmax and staging threads: 0..255
+    const int tiles = (n + Tile::kRows - 1) / Tile::kRows;
+    // staging unit t: rows 4 (t / 4) .. + 3 of the tile, elements 8 (t % 4) .. + 7 of the slice
+    const int quad = t >> 2, piece = t & 3;
+    const bool stager = w > 0 && quad < Tile::kQuads;
+    KvRaw8<KT> reg[4];
+    auto load = [&](int tile) __attribute__((always_inline)) {
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            const int r = min(tile * Tile::kRows + 4 * quad + i, n - 1);  // past the last row: that one, unused
+            reg[i] = kv_raw8<KT>(kv_elem_ptr<KT>(pt_v[r / page_tokens], r % page_tokens, kv_dim, kh * hd + slice * 32), 8 * piece);
+        }
+    };
+    auto store = [&](int buf) __attribute__((always_inline)) {
+#pragma unroll
+        for (int e = 0; e < 8; ++e)
+            *reinterpret_cast<T*>(s_v[buf] + quad * Tile::kPitch + (8 * piece + e) * sizeof(T)) = Rows4<KT>::pack(reg, e);
+    };
+    const float* sr = scores + static_cast<size_t>(h) * n;
+    float mx = -INFINITY;
+    if (w > 0) {
+        const uint64_t tab_v = mvh_expf_tab(t);
+        for (int tt = t; tt < n; tt += kSM) {
+            const float s = sr[tt];
+            s_a[tt] = s;
+            mx = fmaxf(mx, s);
+        }
+        if (stager) load(0);
+        mx = wave_max_all(mx);
+        if ((t & 63) == 0) red_f[t >> 6] = mx;
+        if (t < 32) s_tab[t] = tab_v;
+    }
+    __syncthreads();
+    if (w > 0) {
+        mx = red_f[0];
+#pragma unroll
+        for (int i = 1; i < kSM / 64; ++i) mx = fmaxf(mx, red_f[i]);
+        double den = 0.0;
+        for (int tt = t; tt < n; tt += kSM) {
+            const float e = mvh_expf_tabbed(s_a[tt] - mx, s_tab);
+            s_a[tt] = e;
+            den += static_cast<double>(e);
+        }
+        den = wave_sum(den);
+        if ((t & 63) == 0) red_d[t >> 6] = den;
+        if (stager) {
+            store(0);
+            load(min(1, tiles - 1));
+        }
+    }
+    __syncthreads();
+    if (w > 0) {
+        double den = red_d[0];
+#pragma unroll
+        for (int i = 1; i < kSM / 64; ++i) den += red_d[i];
+        const float inv = static_cast<float>(1.0 / den);
+        for (int tt = t; tt < n; tt += kSM) {
+            float a = s_a[tt] * inv;
+            if constexpr (KT == kKvQ8)
+                a = a * kv_row_scale<KT>(pt_v[tt / page_tokens], tt % page_tokens, page_tokens, kv_dim);
+            s_a[tt] = a;
+        }
+    }
+    __syncthreads();
+    if (w == 0) __builtin_amdgcn_s_setprio(3);  // a stager shares its SIMD
+    float acc = 0.0f;
+    const int d = threadIdx.x & 31;  // the chain's lanes 32..63 repeat 0..31 (not stored)
+    for (int tile = 0; tile < tiles; ++tile) {
+        const int buf = tile & 1;
+        if (w == 0) {
+            const int r0 = tile * Tile::kRows, rows = min(Tile::kRows, n - r0), quads = rows >> 2;
+            const float* pa = s_a + r0;
+            const uint8_t* pv = s_v[buf] + d * sizeof(T);
+            // kQ quads at a time, the next ones read while these are summed
+            constexpr int kQ = KT == kKvF32 ? 4 : 8;
+            float4 wa[2][kQ];
+            T va[2][kQ];
+            const int groups = quads / kQ;
+            auto read = [&](int g, float4 (&ww)[kQ], T (&vv)[kQ]) __attribute__((always_inline)) {
+                g = min(g, groups - 1);
+#pragma unroll
+                for (int i = 0; i < kQ; ++i) {
+                    ww[i] = *reinterpret_cast<const float4*>(pa + 4 * (g * kQ + i));
+                    vv[i] = *reinterpret_cast<const T*>(pv + (g * kQ + i) * Tile::kPitch);
+                }
+            };
+            auto sum = [&](const float4 (&ww)[kQ], const T (&vv)[kQ]) __attribute__((always_inline)) {
+#pragma unroll
+                for (int i = 0; i < kQ; ++i) {
+                    acc = fmaf(ww[i].x, Rows4<KT>::at(vv[i], 0), acc);
+                    acc = fmaf(ww[i].y, Rows4<KT>::at(vv[i], 1), acc);
+                    acc = fmaf(ww[i].z, Rows4<KT>::at(vv[i], 2), acc);
+                    acc = fmaf(ww[i].w, Rows4<KT>::at(vv[i], 3), acc);
+                }
+            };
+            if (groups) {
+                read(0, wa[0], va[0]);
+                int g = 0;
+                for (; g + 2 <= groups; g += 2) {
+                    read(g + 1, wa[1], va[1]);
+                    __builtin_amdgcn_sched_barrier(0);
+                    sum(wa[0], va[0]);
+                    __builtin_amdgcn_sched_barrier(0);
+                    read(g + 2, wa[0], va[0]);
+                    __builtin_amdgcn_sched_barrier(0);
+                    sum(wa[1], va[1]);
+                    __builtin_amdgcn_sched_barrier(0);
+                }
+                if (g < groups) sum(wa[0], va[0]);
+            }
+            for (int r = groups * kQ * 4; r < rows; ++r) {
+                const T v = *reinterpret_cast<const T*>(pv + (r >> 2) * Tile::kPitch);
+                const float x0 = Rows4<KT>::at(v, 0), x1 = Rows4<KT>::at(v, 1), x2 = Rows4<KT>::at(v, 2), x3 = Rows4<KT>::at(v, 3);
+                const int i = r & 3;
+                acc = fmaf(pa[r], i == 0 ? x0 : i == 1 ? x1 : i == 2 ? x2 : x3, acc);
+            }
+        } else if (stager && tile + 1 < tiles) {
+            store(buf ^ 1);  // last read in tile - 1, before the barrier that ended it
+            load(min(tile + 2, tiles - 1));
+        }
+        __syncthreads();
+    }
+    if (threadIdx.x < 32) out[static_cast<size_t>(h) * hd + slice * 32 + d] = acc;
+}
+
+template <int KT>
+hipError_t attn_decode_typed(const void* const* pt_k, const void* const* pt_v, const float* q, float* scores,
+                             float* out, int n, int n_head, int group, int hd, int kv_dim, int page_tokens,
+                             hipStream_t st) {
+    const dim3 gs(static_cast<unsigned>(n_head), static_cast<unsigned>((n + 63) / 64));
+    const size_t lds = static_cast<size_t>(hd) * sizeof(float);
+    if (hd == 128)
+        attn_decode_scores_kernel<KT, 128><<<gs, 64, lds, st>>>(pt_k, q, scores, n, group, hd, kv_dim, page_tokens);
+    else if (hd == 64)
+        attn_decode_scores_kernel<KT, 64><<<gs, 64, lds, st>>>(pt_k, q, scores, n, group, hd, kv_dim, page_tokens);
+    else
+        attn_decode_scores_kernel<KT, 0><<<gs, 64, lds, st>>>(pt_k, q, scores, n, group, hd, kv_dim, page_tokens);
+    if (hipError_t e = hipGetLastError(); e != hipSuccess) return e;
+    attn_decode_v_kernel<KT><<<dim3(static_cast<unsigned>(n_head), static_cast<unsigned>(hd / 32)), kDvThreads,
+                               static_cast<size_t>(n + 3) / 4 * 4 * sizeof(float), st>>>(pt_v, scores, out, n, group,
+                                                                                         hd, kv_dim, page_tokens);
+    return hipGetLastError();
+}
+// weights and V tiles within 64 KB of LDS
+template <int KT>
+bool attn_decode_fits(size_t n) {
+    return (n + 3) / 4 * 4 * sizeof(float) + 2 * DvTile<KT>::kBytes + 512 <= 64 * 1024;
+}
+
 }  // namespace
 
 hipError_t launch_kv_write(int kv_type, void* const* pt_k, void* const* pt_v, const float* k, const float* v,
@@ -1333,7 +1607,17 @@ hipError_t launch_attn_prefill(int kv_type, const void* const* pt_k, const void*
 hipError_t launch_attn_decode(int kv_type, const void* const* pt_k, const void* const* pt_v, const float* q,
                               float* scores, float* out, size_t pos, size_t n_head, size_t n_head_kv, size_t hd,
                               size_t kv_dim, size_t page_tokens, hipStream_t st) {
-    if (hd % 32 == 0)  // V tiles staged in LDS by whole workgroups (latency-bound otherwise)
+    const int n = static_cast<int>(pos + 1), heads = static_cast<int>(n_head), group = static_cast<int>(n_head / n_head_kv);
+    const int d = static_cast<int>(hd), kvd = static_cast<int>(kv_dim), pt = static_cast<int>(page_tokens);
+    if (hd % 32 == 0 && hd <= 512) {
+        if (kv_type == kKvF32 && attn_decode_fits<kKvF32>(pos + 1))
+            return attn_decode_typed<kKvF32>(pt_k, pt_v, q, scores, out, n, heads, group, d, kvd, pt, st);
+        if (kv_type == kKvF16 && attn_decode_fits<kKvF16>(pos + 1))
+            return attn_decode_typed<kKvF16>(pt_k, pt_v, q, scores, out, n, heads, group, d, kvd, pt, st);
+        if (kv_type == kKvQ8 && attn_decode_fits<kKvQ8>(pos + 1))
+            return attn_decode_typed<kKvQ8>(pt_k, pt_v, q, scores, out, n, heads, group, d, kvd, pt, st);
+    }
+    if (hd % 32 == 0)  // weights past the LDS: V tiles staged by whole workgroups
         return launch_attn_prefill(kv_type, pt_k, pt_v, q, n_head * hd, scores, out, nullptr, nullptr, false, nullptr,
                                    pos, pos + 1, 1, n_head, n_head_kv, hd, kv_dim, page_tokens, st);
     return launch_attn(kv_type, pt_k, pt_v, q, n_head * hd, scores, out, nullptr, pos, pos + 1, 1, n_head, n_head_kv,

@@ -687,7 +687,7 @@ __global__ __launch_bounds__(T) void gemv_q6_k_kernel(const uint8_t* __restrict_
     }
 }
 
-// Q6_K for whole groups of 16 tokens on the f64 matrix pipe
+// Q6_K for groups of up to 16 tokens on the f64 matrix pipe
 // (v_mfma_f64_16x16x4f64): the same exact products ((d*sc)*q)*x in double
 // as dot_q6_k_fp32 (src/gguf_kernels.cpp:138-146), accumulated by the
 // MFMA in double.  A workgroup covers 16 rows x 16 tokens; its kQ6FWaves
@@ -710,15 +710,16 @@ typedef double v4f64 __attribute__((ext_vector_type(4)));
 
 __global__ __launch_bounds__(64 * kQ6FWaves) void gemv_q6_k_batch_f64_kernel(const uint8_t* __restrict__ W,
                                                                              const float* __restrict__ x,
-                                                                             float* __restrict__ y, int N, int K) {
+                                                                             float* __restrict__ y, int N, int K,
+                                                                             int B) {
     __shared__ v4f64 s_red[kQ6FWaves][64];
     const int nsb = K / 256;
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     const int li = lane & 15, g = lane >> 4, half = g >> 1, hg = g & 1;
     const int r0 = blockIdx.x * 16, t0 = blockIdx.y * 16;
-    // rows past N use row N - 1 (not written)
+    // rows past N use row N - 1, tokens past B token B - 1 (not written)
     const uint8_t* rb = W + static_cast<size_t>(min(r0 + li, N - 1)) * nsb * 210;
-    const float* xt = x + static_cast<size_t>(t0 + li) * K + 128 * half + 16 * hg;
+    const float* xt = x + static_cast<size_t>(min(t0 + li, B - 1)) * K + 128 * half + 16 * hg;
     const int s_beg = wave * nsb / kQ6FWaves, s_end = (wave + 1) * nsb / kQ6FWaves;
     struct Raw {
         uint32_t qa[4], qb[4], qh[4];
@@ -799,7 +800,7 @@ __global__ __launch_bounds__(64 * kQ6FWaves) void gemv_q6_k_batch_f64_kernel(con
 #pragma unroll
         for (int r = 0; r < 4; ++r) {
             const int row = r0 + 4 * r + g;
-            if (row < N) y[static_cast<size_t>(t0 + li) * N + row] = static_cast<float>(tot[r]);
+            if (row < N && t0 + li < B) y[static_cast<size_t>(t0 + li) * N + row] = static_cast<float>(tot[r]);
         }
     }
 }
@@ -1064,13 +1065,19 @@ size_t gemv_decode_rows_per_wg(uint32_t type, size_t rows, size_t cols) {
 hipError_t launch_gemv_q6_k(const uint8_t* W, const float* x, float* y, size_t rows, size_t cols, size_t batch,
                             hipStream_t st) {
     if (!rows || !batch) return hipSuccess;
-    if (batch >= kQ6BTok) {
-        // whole groups of kQ6BTok tokens on the batch kernel, the rest per token below
-        const size_t groups = batch / kQ6BTok;
+    // Token groups of 16 on the f64 matrix pipe: whole ones, a last one of 5 or
+    // more beside them (5632->2048 at 21 / 117 tokens 38 -> 22 / 85 -> 68 us
+    // against one token at a time for the rest; 3 more than 32 33 -> 37), and 6
+    // or 9 tokens alone (11008->4096 at 6 57 -> 39, 2048->2048 at 6 / 12 6.5 /
+    // 11.0 -> 8.7 / 8.9).
+    const size_t whole = batch / kQ6BTok, left = batch % kQ6BTok;
+    const size_t min_left = whole ? 5 : rows * cols >= (size_t{8} << 20) ? 6 : 9;
+    const size_t groups = whole + (left >= min_left ? 1 : 0);
+    if (groups) {
+        const size_t done = std::min(batch, groups * kQ6BTok);
         const dim3 bgrid(static_cast<unsigned>((rows + kQ6BRows - 1) / kQ6BRows), static_cast<unsigned>(groups));
         gemv_q6_k_batch_f64_kernel<<<bgrid, 64 * kQ6FWaves, 0, st>>>(W, x, y, static_cast<int>(rows),
-                                                                     static_cast<int>(cols));
-        const size_t done = groups * kQ6BTok;
+                                                                     static_cast<int>(cols), static_cast<int>(done));
         if (done == batch) return hipGetLastError();
         x += done * cols;
         y += done * rows;

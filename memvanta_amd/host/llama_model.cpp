@@ -161,7 +161,10 @@ LlamaModel::LlamaModel(const std::string& path, int device, std::size_t ctx_over
     check(hipMemcpy(pt_k_, tk.data(), tk.size() * sizeof(void*), hipMemcpyHostToDevice), "page table");
     check(hipMemcpy(pt_v_, tv.data(), tv.size() * sizeof(void*), hipMemcpyHostToDevice), "page table");
 
-    step_tokens_ = std::max(max_batch_, std::min<std::size_t>(kStepTokens, c_.n_ctx));
+    // a lane's scores stay within 512 MB however long the context
+    step_tokens_ = std::min<std::size_t>(kStepTokens, c_.n_ctx);
+    while (step_tokens_ > 32 && step_tokens_ * c_.n_head * c_.n_ctx * 4 > (std::size_t{512} << 20)) step_tokens_ /= 2;
+    step_tokens_ = std::max(max_batch_, step_tokens_);
     const std::size_t B = step_tokens_, D = c_.n_embd, F = c_.n_ff, KV = c_.kv_dim(), W = std::max(D, F);
     for (Lane& l : lanes_) {
         if (&l != &lanes_[0]) check(hipStreamCreateWithFlags(&l.st, hipStreamNonBlocking), "hipStreamCreate");

@@ -20,6 +20,8 @@ constexpr unsigned kWarmWgs = 256;
 // q8_op_bytes(rows, cols) bytes), else row-major
 hipError_t launch_quantize_q8(const float* x, int8_t* q, float* d, int* s, size_t rows, size_t cols, hipStream_t st,
                               bool q_op = false);
+// n dwords from pinned host memory to device memory (4-byte aligned both)
+hipError_t launch_copy_words(const void* src, void* dst, size_t n, hipStream_t st);
 hipError_t launch_f2h(const float* x, uint16_t* out, size_t n, hipStream_t st);
 hipError_t launch_f2h_bits(uint32_t first, uint16_t* out, size_t n, hipStream_t st);
 hipError_t launch_h2f(const uint16_t* h, float* out, size_t n, hipStream_t st);

@@ -31,6 +31,11 @@ __global__ __launch_bounds__(256) void quantize_q8_kernel(const float4* __restri
     }
 }
 
+__global__ void copy_words_kernel(const uint32_t* __restrict__ src, uint32_t* __restrict__ dst, size_t n) {
+    const size_t i = static_cast<size_t>(blockIdx.x) * blockDim.x + threadIdx.x;
+    if (i < n) dst[i] = src[i];
+}
+
 // fp32_to_fp16 (src/gguf_kernels.cpp:242) over an array.
 __global__ __launch_bounds__(256) void f2h_kernel(const float* __restrict__ x, uint16_t* __restrict__ out, size_t n) {
     const size_t i = static_cast<size_t>(blockIdx.x) * blockDim.x + threadIdx.x;
@@ -94,6 +99,13 @@ hipError_t launch_quantize_q8(const float* x, int8_t* q, float* d, int* s, size_
     const unsigned grid = static_cast<unsigned>((n4 + 255) / 256);
     quantize_q8_kernel<<<grid, 256, 0, st>>>(reinterpret_cast<const float4*>(x), reinterpret_cast<uint32_t*>(q), d,
                                              s, n4, q_op ? static_cast<int>(cols) : 0);
+    return hipGetLastError();
+}
+
+hipError_t launch_copy_words(const void* src, void* dst, size_t n, hipStream_t st) {
+    if (!n) return hipSuccess;
+    copy_words_kernel<<<static_cast<unsigned>((n + 255) / 256), 256, 0, st>>>(static_cast<const uint32_t*>(src),
+                                                                              static_cast<uint32_t*>(dst), n);
     return hipGetLastError();
 }
 

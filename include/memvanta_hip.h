@@ -251,8 +251,8 @@ int mvh_model_reset(mvh_model* m);
 /* LlamaModel::forward: one decode step; logits (host, vocab floats) may be NULL */
 int mvh_model_forward(mvh_model* m, int token, float* logits);
 /* LlamaModel::prefill: chunks of `batch`; logits of the last token when logits != NULL.  Consecutive chunks
- * run on three internal streams (chunk c + 1's layer l beside chunk c's layer l + 1, results identical to a
- * chunk-by-chunk run); every stream is drained before the call returns, also when a later chunk's error is
+ * that give the same bits together join into steps of up to 256 tokens, which run on three internal streams
+ * (step c + 1's layer l beside step c's layer l + 1, results identical to a chunk-by-chunk run); every stream is drained before the call returns, also when a later chunk's error is
  * returned after the earlier chunks completed */
 int mvh_model_prefill(mvh_model* m, const int* tokens, size_t n, size_t batch, float* logits);
 /* n greedy decode steps from `token`, run on the device from one HIP graph (the argmax of each step

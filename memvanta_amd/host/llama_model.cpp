@@ -166,22 +166,34 @@ LlamaModel::LlamaModel(const std::string& path, int device, std::size_t ctx_over
     while (step_tokens_ > 32 && step_tokens_ * c_.n_head * c_.n_ctx * 4 > (std::size_t{512} << 20)) step_tokens_ /= 2;
     step_tokens_ = std::max(max_batch_, step_tokens_);
     const std::size_t B = step_tokens_, D = c_.n_embd, F = c_.n_ff, KV = c_.kv_dim(), W = std::max(D, F);
-    for (Lane& l : lanes_) {
+    for (Lane& l : lanes_)
         if (&l != &lanes_[0]) check(hipStreamCreateWithFlags(&l.st, hipStreamNonBlocking), "hipStreamCreate");
-        l.x = static_cast<float*>(dalloc(B * D * 4));
-        l.n = static_cast<float*>(dalloc(B * D * 4));
-        l.qkv = static_cast<float*>(dalloc(B * (D + 2 * KV) * 4));
-        l.att = static_cast<float*>(dalloc(B * D * 4));
-        l.proj = static_cast<float*>(dalloc(B * D * 4));
-        l.gu = static_cast<float*>(dalloc(B * 2 * F * 4));
-        l.ff = static_cast<float*>(dalloc(B * F * 4));
-        l.scores = static_cast<float*>(dalloc(B * c_.n_head * c_.n_ctx * 4));
-        l.ffo = static_cast<float*>(dalloc(B * D * 4));
-        l.q8 = static_cast<int8_t*>(dalloc(mvh::q8_op_bytes(B, W)));  // row-major or operand order
-        l.q8d = static_cast<float*>(dalloc(B * (W / 32) * 4));
-        l.q8s = static_cast<int8_t*>(dalloc(mvh::q8_op_bytes(B, W)));
-        l.q8sd = static_cast<float*>(dalloc(B * (W / 32) * 4));
-        l.q8ss = static_cast<int*>(dalloc(B * (W / 32) * 4));
+    // the lanes' buffers in one allocation: counted, then carved
+    std::size_t lane_bytes = 0;
+    for (const bool carve : {false, true}) {
+        uint8_t* const slab = carve ? static_cast<uint8_t*>(dalloc(lane_bytes)) : nullptr;
+        lane_bytes = 0;
+        auto take = [&](std::size_t bytes) -> void* {
+            const std::size_t at = lane_bytes;
+            lane_bytes += (std::max<std::size_t>(bytes, 16) + 255) / 256 * 256;
+            return carve ? slab + at : nullptr;
+        };
+        for (Lane& l : lanes_) {
+            l.x = static_cast<float*>(take(B * D * 4));
+            l.n = static_cast<float*>(take(B * D * 4));
+            l.qkv = static_cast<float*>(take(B * (D + 2 * KV) * 4));
+            l.att = static_cast<float*>(take(B * D * 4));
+            l.proj = static_cast<float*>(take(B * D * 4));
+            l.gu = static_cast<float*>(take(B * 2 * F * 4));
+            l.ff = static_cast<float*>(take(B * F * 4));
+            l.scores = static_cast<float*>(take(B * c_.n_head * c_.n_ctx * 4));
+            l.ffo = static_cast<float*>(take(B * D * 4));
+            l.q8 = static_cast<int8_t*>(take(mvh::q8_op_bytes(B, W)));  // row-major or operand order
+            l.q8d = static_cast<float*>(take(B * (W / 32) * 4));
+            l.q8s = static_cast<int8_t*>(take(mvh::q8_op_bytes(B, W)));
+            l.q8sd = static_cast<float*>(take(B * (W / 32) * 4));
+            l.q8ss = static_cast<int*>(take(B * (W / 32) * 4));
+        }
     }
     kv_done_.assign(kLanes * c_.n_layer, nullptr);
     for (hipEvent_t& e : kv_done_) check(hipEventCreateWithFlags(&e, hipEventDisableTiming), "hipEventCreate");

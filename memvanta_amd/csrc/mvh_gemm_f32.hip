@@ -17,6 +17,8 @@
 //   batch_blocksum_kernel  dot_q4_0_fp32 / dot_q8_0_fp32 (:93-120): per block
 //       t_e from zero, s = 0+t0+..+t7, then sum = fma(d, s, sum) over the blocks.
 #include "mvh_kernels.hpp"
+#define MVH_STAGE_QUAL __device__ __forceinline__
+#include "mvh_stage.h"
 
 #include <cstdlib>
 #include <type_traits>
@@ -68,7 +70,7 @@ __device__ __forceinline__ T ld_at(const void* base, uint32_t off) {
 // Bytes of blocks [c*8, c*8+8) of 16*R rows into registers, and from there to
 // an LDS copy of pitch kUB bytes per row.  ALIGNED (K % 256 == 0: a row's unit
 // starts 16-byte aligned): 16-byte pieces.  Otherwise 2-byte pieces, those past
-// the row's last block left out.
+// the row's last block read from its start (mvh_stage.h).
 template <uint32_t TYPE, int R, bool ALIGNED>
 struct WStage {
     static constexpr int kUB = kUnitBlocks * Fmt<TYPE>::kB;
@@ -78,27 +80,21 @@ struct WStage {
     static constexpr int kN = (kRows * kP + kT - 1) / kT;
     typedef std::conditional_t<ALIGNED, uint4, uint16_t> Piece;
     const uint8_t* base;       // the tile's first row (uniform)
-    uint32_t src[kN];          // byte offset of piece i in unit 0
-    int dst[kN], off[kN];
+    MvhStagePiece src[kN];
+    int dst[kN];
     __device__ __forceinline__ void init(const uint8_t* W, int row0, int N, int row_bytes) {
         base = W + static_cast<size_t>(row0) * row_bytes;
 #pragma unroll
         for (int i = 0; i < kN; ++i) {
-            const int p = static_cast<int>(threadIdx.x) + kT * i, pc = min(p, kRows * kP - 1);
-            off[i] = static_cast<int>(sizeof(Piece)) * (pc % kP);
-            // rows past N read row N - 1 (their results are not stored)
-            src[i] = static_cast<uint32_t>(min(pc / kP, N - 1 - row0)) * static_cast<uint32_t>(row_bytes) + off[i];
-            dst[i] = p < kRows * kP ? (pc / kP) * kUB + off[i] : kRows * kUB;
+            const int p = static_cast<int>(threadIdx.x) + kT * i;
+            src[i] = mvh_stage_piece(p, kRows * kP, kP, sizeof(Piece), N - row0, row_bytes);
+            dst[i] = p < kRows * kP ? (p / kP) * kUB + src[i].off : kRows * kUB;
         }
     }
     __device__ __forceinline__ void load(int i, int c, int row_bytes, Piece (&reg)[kN]) const {
         const int at = c * kUB;
-        if constexpr (ALIGNED) {
-            reg[i] = ld_at<uint4>(base + at, src[i]);
-        } else {
-            const int lim = at + off[i] < row_bytes ? at : 0;  // past the row: any byte of it, unused
-            reg[i] = ld_at<uint16_t>(base, src[i] + lim);
-        }
+        if constexpr (ALIGNED) reg[i] = ld_at<uint4>(base + at, src[i].src);
+        else reg[i] = ld_at<uint16_t>(base, mvh_stage_at(src[i], at, row_bytes));
     }
     __device__ __forceinline__ void store(int i, uint8_t* s, const Piece (&reg)[kN]) const {
         *reinterpret_cast<Piece*>(s + dst[i]) = reg[i];

@@ -1062,19 +1062,22 @@ size_t gemv_decode_rows_per_wg(uint32_t type, size_t rows, size_t cols) {
     return 0;
 }
 
+// Token groups of 16 on the f64 matrix pipe: whole ones, a last one of 5 or
+// more beside them (5632->2048 at 21 / 117 tokens 38 -> 22 / 85 -> 68 us
+// against one token at a time for the rest; 3 more than 32 33 -> 37), and 6
+// or 9 tokens alone (11008->4096 at 6 57 -> 39, 2048->2048 at 6 / 12 6.5 /
+// 11.0 -> 8.7 / 8.9).
+size_t gemv_q6_k_group_tokens(size_t rows, size_t cols, size_t batch) {
+    const size_t whole = batch / kQ6BTok, left = batch % kQ6BTok;
+    const size_t min_left = whole ? 5 : rows * cols >= (size_t{8} << 20) ? 6 : 9;
+    return left >= min_left ? batch : whole * kQ6BTok;
+}
+
 hipError_t launch_gemv_q6_k(const uint8_t* W, const float* x, float* y, size_t rows, size_t cols, size_t batch,
                             hipStream_t st) {
     if (!rows || !batch) return hipSuccess;
-    // Token groups of 16 on the f64 matrix pipe: whole ones, a last one of 5 or
-    // more beside them (5632->2048 at 21 / 117 tokens 38 -> 22 / 85 -> 68 us
-    // against one token at a time for the rest; 3 more than 32 33 -> 37), and 6
-    // or 9 tokens alone (11008->4096 at 6 57 -> 39, 2048->2048 at 6 / 12 6.5 /
-    // 11.0 -> 8.7 / 8.9).
-    const size_t whole = batch / kQ6BTok, left = batch % kQ6BTok;
-    const size_t min_left = whole ? 5 : rows * cols >= (size_t{8} << 20) ? 6 : 9;
-    const size_t groups = whole + (left >= min_left ? 1 : 0);
-    if (groups) {
-        const size_t done = std::min(batch, groups * kQ6BTok);
+    if (const size_t done = gemv_q6_k_group_tokens(rows, cols, batch)) {
+        const size_t groups = (done + kQ6BTok - 1) / kQ6BTok;
         const dim3 bgrid(static_cast<unsigned>((rows + kQ6BRows - 1) / kQ6BRows), static_cast<unsigned>(groups));
         gemv_q6_k_batch_f64_kernel<<<bgrid, 64 * kQ6FWaves, 0, st>>>(W, x, y, static_cast<int>(rows),
                                                                      static_cast<int>(cols), static_cast<int>(done));

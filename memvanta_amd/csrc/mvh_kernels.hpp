@@ -38,6 +38,9 @@ hipError_t launch_gemv_q8_0(const uint8_t* W, const float* x, float* y, size_t r
                             hipStream_t st);
 hipError_t launch_gemv_q6_k(const uint8_t* W, const float* x, float* y, size_t rows, size_t cols, size_t batch,
                             hipStream_t st);
+// the leading tokens of a Q6_K batch that take the f64 matrix pipe; the rest go
+// one at a time, which adds the same doubles in another order
+size_t gemv_q6_k_group_tokens(size_t rows, size_t cols, size_t batch);
 // F32 / F16 weights with fp32 activations, y[b*rows + r] (dot_f32_simd / the double F16 sum)
 hipError_t launch_gemv_f32(const float* W, const float* x, float* y, size_t rows, size_t cols, size_t batch,
                            hipStream_t st);

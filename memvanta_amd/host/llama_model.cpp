@@ -122,6 +122,11 @@ LlamaModel::LlamaModel(const std::string& path, int device, std::size_t ctx_over
             rows(L.gate_up, L.gate) != (L.fused_gu ? 2 * c_.n_ff : c_.n_ff) || L.down.rows != c_.n_embd ||
             L.down.cols != c_.n_ff)
             throw std::runtime_error("layer " + std::to_string(i) + ": weight shapes do not match the config");
+        for (const Tensor* t : {&L.qkv, &L.q, &L.k, &L.v, &L.o, &L.gate_up, &L.gate, &L.up, &L.down}) {
+            const std::pair<std::size_t, std::size_t> shape{t->rows, t->cols};
+            if (t->d && t->type == 14 && std::find(q6k_shapes_.begin(), q6k_shapes_.end(), shape) == q6k_shapes_.end())
+                q6k_shapes_.push_back(shape);
+        }
     }
 
     // RoPE table computed on the host with the C library, as the reference
@@ -646,15 +651,24 @@ const char* LlamaModel::chunk_error(const std::vector<int>& tokens, std::size_t 
     return nullptr;
 }
 
-// Whether consecutive chunks of `batch` tokens (and a last one of 2 or more)
-// give the same bits in one step.  A token's results depend on its chunk only
-// through the arithmetic the chunk's size selects for it: in the fp32
-// numerics the last B % 8 (feed-forward) or B % 4 tokens of a chunk take the
-// per-token dots, so whole multiples of 8 join, and the last chunk's leftover
-// tokens are the joined step's; in the Q8 numerics every token of a chunk of
-// 2 or more is treated alike (one of 1 has its own path).
-bool LlamaModel::chunks_join(std::size_t batch) const {
-    return mode_ == PrefillMode::Q8 ? batch >= 2 : batch % 8 == 0;
+// Whether a step of B tokens (whole chunks of `batch`) and the chunk of `next`
+// tokens after it give the same bits in one step.  A token's results depend on
+// its chunk only through the arithmetic the chunk's size selects for it:
+//   * a chunk of 1 has a path of its own;
+//   * in the fp32 numerics the last B % 8 (feed-forward) or B % 4 tokens of a
+//     chunk take the per-token dots, so whole multiples of 8 join, and the last
+//     chunk's leftover tokens are the joined step's; in the Q8 numerics every
+//     token is treated alike;
+//   * Q6_K weights take a chunk's leading tokens to the f64 matrix pipe and the
+//     rest one at a time, with another order of the sums: each token has to be
+//     on the same side of that line as in its own chunk.
+bool LlamaModel::chunks_join(std::size_t batch, std::size_t B, std::size_t next) const {
+    if (next < 2 || (mode_ == PrefillMode::Q8 ? batch < 2 : batch % 8 != 0)) return false;
+    for (const auto& [rows, cols] : q6k_shapes_)
+        if (mvh::gemv_q6_k_group_tokens(rows, cols, B) != B ||
+            mvh::gemv_q6_k_group_tokens(rows, cols, B + next) != B + mvh::gemv_q6_k_group_tokens(rows, cols, next))
+            return false;
+    return true;
 }
 
 const std::vector<float>& LlamaModel::prefill(const std::vector<int>& tokens, std::size_t batch_size,
@@ -689,9 +703,9 @@ const std::vector<float>& LlamaModel::prefill(const std::vector<int>& tokens, st
             // the chunks before a refused one complete (drained below)
             if (const char* err = chunk_error(tokens, i, B)) throw std::runtime_error(err);
             // later chunks join the step while that leaves every result as it is
-            while (!profiling_ && i + B < tokens.size() && chunks_join(batch_size)) {
+            while (!profiling_ && i + B < tokens.size()) {
                 const std::size_t next = std::min(batch_size, tokens.size() - i - B);
-                if (next < 2 || B + next > step_tokens_ || chunk_error(tokens, i, B + next)) break;
+                if (!chunks_join(batch_size, B, next) || B + next > step_tokens_ || chunk_error(tokens, i, B + next)) break;
                 B += next;
             }
             const bool last = compute_logits_last && i + B == tokens.size();

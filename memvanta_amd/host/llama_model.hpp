@@ -12,6 +12,7 @@
 #include <cstdint>
 #include <memory>
 #include <string>
+#include <utility>
 #include <vector>
 
 #include "profile.hpp"
@@ -91,7 +92,7 @@ private:
     void store_kv(const QkvLayout& lay, void* const* pk, void* const* pv, const int* d_pos, std::size_t pos,
                   std::size_t B);
     const char* chunk_error(const std::vector<int>& tokens, std::size_t i, std::size_t B) const;
-    bool chunks_join(std::size_t batch) const;
+    bool chunks_join(std::size_t batch, std::size_t B, std::size_t next) const;
     // one prefill step (a chunk, or consecutive ones joined) on lane ln_;
     // prev_lane >= 0: the previous step runs on that lane and this step's
     // attention of layer l waits for its KV of layer l
@@ -131,6 +132,7 @@ private:
     Tensor embd_, out_;
     float* out_norm_{};
     std::vector<Layer> layers_;
+    std::vector<std::pair<std::size_t, std::size_t>> q6k_shapes_;  // (rows, cols) of the layers' Q6_K weights, each once
     std::vector<void*> allocs_;
     // paged KV: one slab per kind, page tables per layer ([layer][max_pages])
     void** pt_k_{};

@@ -72,3 +72,56 @@ def test_later_rows_do_not_reach_earlier_tokens(ctx, kv_type, B):
         kv.close()
     a, b = (o[: B - 3].view(np.uint32) for o in outs)
     assert (a == b).all()
+
+
+def _joined_equals_single(path, mode, kv_type, n, batch, vocab):
+    prompt = np.random.default_rng(n).integers(0, vocab, n).astype(np.int32)
+    m = capi.Model(path, act_mode=mode, max_batch=64, kv_type=kv_type)
+    got = m.prefill(prompt, batch).copy()
+    m.reset()
+    for i in range(0, n, batch):
+        want = m.prefill(prompt[i:i + batch], batch)
+    assert np.isfinite(got).all()
+    assert (got.view(np.uint32) == want.view(np.uint32)).all()
+    m.close()
+
+
+def _order_sensitive(path, monkeypatch):
+    """A layer whose Q6_K q|k|v sums hold two huge terms that cancel (equal weights and embeddings in columns 3 and 300,
+    norm weights +-2^45), so that the order of the double sum shows in the result's leading digits."""
+    cfg = synth.ModelConfig("q6k-sums", 512, 1024, 1, 8, 8, 64, 128, synth.Q6_K, synth.F32, synth.Q6_K)
+    rng = np.random.default_rng(9)
+
+    def content(name, dims):
+        if name == "blk.0.attn_norm.weight":
+            v = np.ones(512, np.float32)
+            v[3], v[300] = 2.0 ** 45, -(2.0 ** 45)
+            return v
+        m = rng.standard_normal((dims[1], 512), dtype=np.float32)
+        if name == "token_embd.weight":
+            m[:, 300] = m[:, 3]
+            return m
+        m = np.clip(m * np.float32(0.02), -0.05, 0.05)
+        m[:, 15::16] = 0.062  # every 16-element scale is the same
+        m[:, 300] = m[:, 3] = 0.04
+        return synth.quantize(synth.Q6_K, m)
+
+    class Writer(synth.GgufWriter):
+        def add_tensor(self, name, dims, ty, nbytes, produce):
+            if name in ("blk.0.attn_norm.weight", "token_embd.weight") or name[6:] in ("attn_q.weight", "attn_k.weight", "attn_v.weight"):
+                b = content(name, dims).tobytes()
+                produce = lambda: iter([b])
+            super().add_tensor(name, dims, ty, nbytes, produce)
+
+    monkeypatch.setattr(synth, "GgufWriter", Writer)
+    synth.write_model(cfg, path, seed=3, digest=False)
+
+
+@pytest.mark.parametrize("mode,n,batch", [(0, 37, 32), (0, 40, 8), (0, 69, 64), (0, 87, 32), (0, 77, 32), (1, 24, 3),
+                                          (1, 50, 20), (1, 72, 24)])
+def test_q6k_sums_keep_their_order(tmp_path, monkeypatch, mode, n, batch):
+    """Q6_K chunks whose tokens go one at a time do not join a step that would group them: last chunks of 5 and 8
+    beside whole groups, chunks of 3 and 8, 20 (16 and 4); 23, 13 and 24 tokens are grouped alone as in a step."""
+    path = str(tmp_path / "q6k.gguf")
+    _order_sensitive(path, monkeypatch)
+    _joined_equals_single(path, mode, capi.MVH_KV_F16, n, batch, 64)

@@ -74,6 +74,22 @@ def test_later_rows_do_not_reach_earlier_tokens(ctx, kv_type, B):
     assert (a == b).all()
 
 
+# Shapes whose joined steps leave the fallback kernels: 128-wide heads over Q4_0 (256-token steps of gate|up on the 64-row
+# int8 tiles, scores tiles of more than 32 tokens), and 64-wide grouped heads over Q8_0 with a Q6_K down projection
+_WIDE = synth.ModelConfig("joined-q4", 1024, 2816, 2, 8, 8, 512, 384, synth.Q4_0, synth.Q4_0, synth.Q4_0)
+_GROUPED = synth.ModelConfig("joined-q8-q6", 1024, 2816, 2, 16, 4, 512, 384, synth.Q8_0, synth.Q8_0, synth.Q6_K,
+                             synth.Q6_K)
+
+
+@pytest.fixture(scope="module")
+def shapes(tmp_path_factory):
+    out = {}
+    for cfg in (_WIDE, _GROUPED):
+        out[cfg.name] = str(tmp_path_factory.mktemp("joined") / (cfg.name + ".gguf"))
+        synth.write_model(cfg, out[cfg.name], seed=5, device="cuda", digest=False)
+    return out
+
+
 def _joined_equals_single(path, mode, kv_type, n, batch, vocab):
     prompt = np.random.default_rng(n).integers(0, vocab, n).astype(np.int32)
     m = capi.Model(path, act_mode=mode, max_batch=64, kv_type=kv_type)
@@ -84,6 +100,15 @@ def _joined_equals_single(path, mode, kv_type, n, batch, vocab):
     assert np.isfinite(got).all()
     assert (got.view(np.uint32) == want.view(np.uint32)).all()
     m.close()
+
+
+@pytest.mark.parametrize("name,mode,kv,n,batch", [
+    ("joined-q4", 1, capi.MVH_KV_F16, 300, 32), ("joined-q4", 1, capi.MVH_KV_Q8, 261, 16),
+    ("joined-q4", 0, capi.MVH_KV_F32, 275, 8), ("joined-q4", 0, capi.MVH_KV_F16, 230, 64),
+    ("joined-q8-q6", 0, capi.MVH_KV_F16, 300, 32), ("joined-q8-q6", 0, capi.MVH_KV_Q8, 261, 32),
+    ("joined-q8-q6", 1, capi.MVH_KV_F16, 90, 5), ("joined-q8-q6", 1, capi.MVH_KV_F32, 77, 24)])
+def test_joined_equals_single_chunks_wide(shapes, name, mode, kv, n, batch):
+    _joined_equals_single(shapes[name], mode, kv, n, batch, 512)
 
 
 def _order_sensitive(path, monkeypatch):

@@ -5,9 +5,11 @@
 #include "memvanta_hip.h"
 #include "mvh_kernels.hpp"
 #include "llama_model.hpp"
+#include "pin_pool.hpp"
 #include "profile.hpp"
 
 #include <algorithm>
+#include <atomic>
 #include <cstdarg>
 #include <cstdio>
 #include <cstring>
@@ -28,8 +30,10 @@ struct mvh_context {
     Buf xin;      // host-pointer staging of inputs
     Buf yout;     // host-pointer staging of outputs
     Buf scores;   // attention scores
-    // pinned host memory of the one-token calls with host vectors: the first
-    // kPinIn bytes for the input, kPinOut for the output (made by the first such call)
+    // pinned host memory of a one-token call with host vectors: the first
+    // kPinIn bytes for the input, kPinOut for the output.  Borrowed for the
+    // call; kept where the call failed with work perhaps still in flight, or
+    // the pool was full.
     uint8_t* pin = nullptr;
     static constexpr size_t kPinIn = 64 << 10, kPinOut = 256 << 10;
 };
@@ -169,18 +173,37 @@ int finish_out(mvh_context* c, void* host_dst, const void* dev_src, size_t bytes
 
 // One-token calls with host vectors: pageable copies cost a staging copy and a
 // wait each way, so the input goes through pinned memory and a copy kernel,
-// and the GEMV stores its rows to pinned memory itself.  Each call ends with
-// the stream drained, so the memory is free for the next one.  Q4_0
-// 4096->11008 35.5 -> 25.6 us a call (the first of a context 80 -> 110).
+// and the GEMV stores its rows to pinned memory itself.  A call ends with the
+// stream drained and its block given back, so contexts share the blocks and
+// only calls that overlap make more.  Against the staged copies (us a call):
+// Q4_0 288->288 32 -> 22.5, 4096->11008 35 -> 25, 512->60000 53.5 -> 44; Q8_0
+// 2048->5632 31 -> 21.4, 256->65536 41.5 -> 31; Q6_K 4096->32000 58 -> 47; F16
+// 4096->4096 48 -> 39; F32 2048->2048 65 -> 54.  A context's first call takes
+// 1 us more than its later ones (10-20 us with a block of its own).
+struct PinAlloc {
+    static uint8_t* make() {
+        uint8_t* p = nullptr;
+        if (hipHostMalloc(reinterpret_cast<void**>(&p), mvh_context::kPinIn + mvh_context::kPinOut,
+                          hipHostMallocPortable) == hipSuccess)
+            return p;
+        (void)hipGetLastError();
+        return nullptr;
+    }
+    static void drop(uint8_t* p) { (void)hipHostFree(p); }
+};
+constexpr size_t kPinKept = 8;   // 2.5 MB
+std::atomic<int> g_contexts{0};  // with the last context all free blocks but one go
+memvanta::hip::PinPool<PinAlloc>& pins() {
+    static auto* const p = new memvanta::hip::PinPool<PinAlloc>(kPinKept);  // outlives the HIP runtime's own teardown
+    return *p;
+}
 bool pin_ready(mvh_context* c, size_t in, size_t out) {
     if (in > mvh_context::kPinIn || out > mvh_context::kPinOut) return false;
-    if (!c->pin &&
-        hipHostMalloc(reinterpret_cast<void**>(&c->pin), mvh_context::kPinIn + mvh_context::kPinOut, hipHostMallocDefault) !=
-            hipSuccess) {
-        (void)hipGetLastError();
-        c->pin = nullptr;
-    }
+    if (!c->pin) c->pin = pins().take();
     return c->pin != nullptr;
+}
+void pin_done(mvh_context* c) {
+    if (c->pin && pins().give(c->pin)) c->pin = nullptr;
 }
 
 // Q8 activation scratch: q [rows][cols] | d [rows][cols/32] | s [rows][cols/32]
@@ -360,6 +383,7 @@ int mvh_context_create(int device, mvh_context** out) {
         delete c;
         return fail(MVH_E_DEVICE, "hipStreamCreate failed");
     }
+    ++g_contexts;
     *out = c;
     return MVH_OK;
 }
@@ -367,10 +391,11 @@ int mvh_context_create(int device, mvh_context** out) {
 int mvh_context_destroy(mvh_context* c) {
     if (!c) return MVH_OK;
     (void)hipSetDevice(c->device);
-    (void)hipStreamSynchronize(c->stream);
+    if (hipStreamSynchronize(c->stream) == hipSuccess) pin_done(c);
     for (auto* b : {&c->act, &c->xin, &c->yout, &c->scores})
         if (b->p) (void)hipFree(b->p);
     if (c->pin) (void)hipHostFree(c->pin);
+    if (--g_contexts == 0) pins().trim(1);
     (void)hipStreamDestroy(c->stream);
     delete c;
     return MVH_OK;
@@ -545,6 +570,7 @@ int mvh_matvec(mvh_context* c, const mvh_tensor* w, const float* x, float* y, in
     if (pinned) {
         MVH_HIP(hipStreamSynchronize(c->stream));
         std::memcpy(y, yd, rows * 4);
+        pin_done(c);
         return MVH_OK;
     }
     return finish_out(c, y, yd, rows * 4, kind);

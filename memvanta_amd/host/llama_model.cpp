@@ -13,6 +13,7 @@
 
 #include "gguf.hpp"
 #include "mvh_kernels.hpp"
+#include "step_plan.hpp"
 
 namespace memvanta {
 namespace hip {
@@ -166,22 +167,23 @@ LlamaModel::LlamaModel(const std::string& path, int device, std::size_t ctx_over
     check(hipMemcpy(pt_k_, tk.data(), tk.size() * sizeof(void*), hipMemcpyHostToDevice), "page table");
     check(hipMemcpy(pt_v_, tv.data(), tv.size() * sizeof(void*), hipMemcpyHostToDevice), "page table");
 
-    // a lane's scores stay within 512 MB however long the context
-    step_tokens_ = std::min<std::size_t>(kStepTokens, c_.n_ctx);
-    while (step_tokens_ > 32 && step_tokens_ * c_.n_head * c_.n_ctx * 4 > (std::size_t{512} << 20)) step_tokens_ /= 2;
-    step_tokens_ = std::max(max_batch_, step_tokens_);
-    const std::size_t B = step_tokens_, D = c_.n_embd, F = c_.n_ff, KV = c_.kv_dim(), W = std::max(D, F);
+    // the small buffers first: the lanes take what is left, down to max_batch_ tokens each
+    const std::size_t most = step_tokens(max_batch_, kStepTokens, c_.n_ctx, c_.n_head, mode_ == PrefillMode::Q8);
+    logits_d_ = static_cast<float*>(dalloc(c_.vocab * 4));
+    d_tok_ = static_cast<int*>(dalloc(16));
+    d_hist_ = static_cast<int*>(dalloc(4 * (c_.n_ctx + 1)));
+    d_pos_ = static_cast<int*>(dalloc(16));
+    d_prompt_ = static_cast<int*>(dalloc(4 * (c_.n_ctx + most)));
+    const std::size_t D = c_.n_embd, F = c_.n_ff, KV = c_.kv_dim(), W = std::max(D, F);
     for (Lane& l : lanes_)
         if (&l != &lanes_[0]) check(hipStreamCreateWithFlags(&l.st, hipStreamNonBlocking), "hipStreamCreate");
     // the lanes' buffers in one allocation: counted, then carved
-    std::size_t lane_bytes = 0;
-    for (const bool carve : {false, true}) {
-        uint8_t* const slab = carve ? static_cast<uint8_t*>(dalloc(lane_bytes)) : nullptr;
-        lane_bytes = 0;
-        auto take = [&](std::size_t bytes) -> void* {
-            const std::size_t at = lane_bytes;
-            lane_bytes += (std::max<std::size_t>(bytes, 16) + 255) / 256 * 256;
-            return carve ? slab + at : nullptr;
+    auto carve = [&](uint8_t* slab, std::size_t B) {
+        std::size_t bytes = 0;
+        auto take = [&](std::size_t n) -> void* {
+            const std::size_t at = bytes;
+            bytes += (std::max<std::size_t>(n, 16) + 255) / 256 * 256;
+            return slab ? slab + at : nullptr;
         };
         for (Lane& l : lanes_) {
             l.x = static_cast<float*>(take(B * D * 4));
@@ -199,16 +201,25 @@ LlamaModel::LlamaModel(const std::string& path, int device, std::size_t ctx_over
             l.q8sd = static_cast<float*>(take(B * (W / 32) * 4));
             l.q8ss = static_cast<int*>(take(B * (W / 32) * 4));
         }
-    }
+        return bytes;
+    };
+    hipError_t lanes_err = hipSuccess;
+    step_tokens_ = fit_step(most, max_batch_, [&](std::size_t B) {
+        void* slab = nullptr;
+        lanes_err = hipMalloc(&slab, carve(nullptr, B));
+        if (lanes_err != hipSuccess) {
+            (void)hipGetLastError();
+            return false;
+        }
+        allocs_.push_back(slab);
+        carve(static_cast<uint8_t*>(slab), B);
+        return true;
+    });
+    check(lanes_err, "hipMalloc");
     kv_done_.assign(kLanes * c_.n_layer, nullptr);
     for (hipEvent_t& e : kv_done_) check(hipEventCreateWithFlags(&e, hipEventDisableTiming), "hipEventCreate");
-    logits_d_ = static_cast<float*>(dalloc(c_.vocab * 4));
-    d_tok_ = static_cast<int*>(dalloc(16));
-    d_hist_ = static_cast<int*>(dalloc(4 * (c_.n_ctx + 1)));
-    d_pos_ = static_cast<int*>(dalloc(16));
-    d_prompt_ = static_cast<int*>(dalloc(4 * (c_.n_ctx + B)));
     rec_ = std::make_unique<prof::Recorder>(lanes_[0].st);
-    check(hipHostMalloc(reinterpret_cast<void**>(&pin_), 4 * (c_.n_ctx + B + 8), hipHostMallocDefault),
+    check(hipHostMalloc(reinterpret_cast<void**>(&pin_), 4 * (c_.n_ctx + most + 8), hipHostMallocDefault),
           "hipHostMalloc");
     logits_.resize(c_.vocab);
     fused_attn_ = kv_type_ == mvh::kKvF16 && mvh::attn_decode_fused_ok(c_.head_dim(), c_.n_ctx, page_tokens_);
@@ -663,7 +674,7 @@ const char* LlamaModel::chunk_error(const std::vector<int>& tokens, std::size_t 
 //     rest one at a time, with another order of the sums: each token has to be
 //     on the same side of that line as in its own chunk.
 bool LlamaModel::chunks_join(std::size_t batch, std::size_t B, std::size_t next) const {
-    if (next < 2 || (mode_ == PrefillMode::Q8 ? batch < 2 : batch % 8 != 0)) return false;
+    if (next < 2 || !batch_joins(batch, mode_ == PrefillMode::Q8)) return false;
     for (const auto& [rows, cols] : q6k_shapes_)
         if (mvh::gemv_q6_k_group_tokens(rows, cols, B) != B ||
             mvh::gemv_q6_k_group_tokens(rows, cols, B + next) != B + mvh::gemv_q6_k_group_tokens(rows, cols, next))

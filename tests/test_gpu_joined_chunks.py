@@ -4,6 +4,7 @@ import dataclasses
 
 import numpy as np
 import pytest
+import torch
 
 from memvanta_amd import capi, synth
 
@@ -53,6 +54,18 @@ def test_joined_equals_single_chunks(tiny, mode, n, batch):
         want = m.prefill(prompt[i:i + batch], batch)
     assert (got.view(np.uint32) == want.view(np.uint32)).all()
     m.close()
+
+
+def test_buffers_of_a_model_that_never_joins(tiny):
+    """In the fp32 numerics chunks of up to 4 tokens never join: buffers for 4, not for a 256-token step (some 20 MB)."""
+    used = {}
+    for max_batch in (8, 4, 8):  # the first one also takes what a process's first model does
+        free = torch.cuda.mem_get_info()[0]
+        m = capi.Model(tiny, ctx=256, act_mode=0, max_batch=max_batch)
+        used[max_batch] = free - torch.cuda.mem_get_info()[0]
+        m.prefill(synth.prompt_tokens(3, 70).astype(np.int32), max_batch)
+        m.close()
+    assert used[4] + (10 << 20) < used[8]
 
 
 @pytest.mark.parametrize("kv_type", [capi.MVH_KV_F32, capi.MVH_KV_F16])
@@ -133,7 +146,8 @@ def _order_sensitive(path, monkeypatch):
 
     class Writer(synth.GgufWriter):
         def add_tensor(self, name, dims, ty, nbytes, produce):
-            if name in ("blk.0.attn_norm.weight", "token_embd.weight") or name[6:] in ("attn_q.weight", "attn_k.weight", "attn_v.weight"):
+            if name in ("token_embd.weight", "blk.0.attn_norm.weight", "blk.0.attn_q.weight", "blk.0.attn_k.weight",
+                        "blk.0.attn_v.weight"):
                 b = content(name, dims).tobytes()
                 produce = lambda: iter([b])
             super().add_tensor(name, dims, ty, nbytes, produce)

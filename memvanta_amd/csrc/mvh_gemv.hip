@@ -955,6 +955,22 @@ static hipError_t launch_f32act(const uint8_t* W, const float* x, float* y, size
     return hipGetLastError();
 }
 
+// Whether several tokens take the f32 matrix pipe (K % 256 == 0), whose 16-row,
+// 16-token tile costs about 2 us per 512 columns however full it is.  The
+// kernels of launch_f32act cost by rows x tokens above a floor, and take 4
+// tokens a workgroup up to K = 2048, 2 up to 4096, then one.  Up to 3 tokens
+// they are even or ahead (4096x4096 Q4_0 at 2 / 3 / 4 tokens 11.6 / 15.6 / 18.3
+// against 17.8 us).  8 tokens, matrix pipe / those (us, Q8_0): 512->64 3.7 / 8.6,
+// 2048->64 9.6 / 10.1; 4096->64 / 768 / 2048 18 / 8.6, 18 / 11.6, 18 / 20;
+// 8192->64 / 1024 / 1536 34 / 7, 34 / 30, 34 / 41; 11008->1024 46 / 79.  4..7
+// tokens beyond K = 4608 want more rows (8192->1536 at 6 34 / 32).
+static bool enough_for_blocksum(size_t rows, size_t cols, size_t batch) {
+    const size_t work = rows * batch;
+    if (cols <= 2048) return true;
+    if (cols <= 4608) return work > (cols <= 3072 ? 5 << 10 : 12 << 10);
+    return work >= 8 << 10 && (batch >= 8 || rows >= 4096);
+}
+
 // One token, K % 256 == 0, K <= 16384: the persistent kernel; otherwise the
 // two-phase kernel per token.
 template <uint32_t TYPE>
@@ -997,14 +1013,8 @@ static hipError_t launch_f32act_any(const uint8_t* W, const float* x, float* y, 
             gemv_f32act_persistent_nq8_0<<<g, 256, lds, st>>>(W, x, y, n, nb, ntiles);
         return hipGetLastError();
     }
-    // Several tokens at K % 256 == 0: the f32 matrix pipe, whose 16-token tile
-    // costs about 2 us per 512 columns however few tokens are in it.  Up to 3
-    // tokens the kernels below are even or ahead (4096x4096 Q4_0 at 2 / 3 / 4
-    // tokens 11.6 / 15.6 / 18.3 against 17.8 us), and at 4..7 tokens for a long
-    // K over few rows, which leaves it too few workgroups (8192->1000 at 5
-    // tokens 22 against 34 us, 11008->4096 194 against 46).
     if constexpr (TYPE == kQ4_0 || TYPE == kQ8_0) {
-        if (batch >= 4 && (batch >= 8 || cols <= 4096 || rows >= 4096) && batch_blocksum_ok(TYPE, W, cols))
+        if (batch >= 4 && enough_for_blocksum(rows, cols, batch) && batch_blocksum_ok(TYPE, W, cols))
             return launch_batch_blocksum(TYPE, W, x, y, rows, cols, batch, st);
     }
     return launch_f32act<TYPE>(W, x, y, rows, cols, batch, st);

@@ -4,6 +4,7 @@ against the oracle at the edges of their tiles.
 Both numerics are fma chains in a fixed order and the kernels run the same chains, so the tolerance is none."""
 import numpy as np
 import pytest
+import torch
 
 from conftest import assert_bitexact
 from memvanta_amd import capi, synth
@@ -45,3 +46,39 @@ def test_block_sums_bitexact(ctx, oracle, ty, batch, k, n):
     if ty == synth.Q8_0:
         assert_bitexact(ctx.matmul_batch_v06(t, x, capi.MVH_ACT_Q8), want, f"v06 q8 B={batch} K={k} N={n}")
     t.free()
+
+
+# rows x tokens on both sides of the lines between the matrix pipe and the per-token kernels: none up to K = 2048, 5 K up
+# to 3072, 12 K up to 4608, 8 K beyond (there with 4096 rows or 8 tokens)
+@pytest.mark.parametrize("ty", [synth.Q4_0, synth.Q8_0])
+@pytest.mark.parametrize("batch,k,n", [(4, 2048, 33), (4, 2304, 1280), (4, 2304, 1281), (5, 3072, 1025),
+                                       (8, 3328, 1536), (8, 3328, 1537), (16, 4608, 769), (8, 4864, 1023),
+                                       (8, 4864, 1024), (7, 8192, 1200), (4, 5120, 4096), (17, 8192, 600)])
+def test_block_sums_where_they_pay_bitexact(ctx, oracle, ty, batch, k, n):
+    test_block_sums_bitexact(ctx, oracle, ty, batch, k, n)
+
+
+@pytest.mark.parametrize("ty,few,many,k", [(synth.Q8_0, 2, 8, 8192), (synth.Q4_0, 2, 11, 8192)])
+def test_few_rows_cost_by_their_tokens(ctx, ty, few, many, k):
+    """A matrix of 64 rows leaves most of the chip idle, so more tokens of it cost next to nothing (1.0 to 1.1 times
+    seen), unless they take a tile whose time is the same however full it is (4 to 5 times)."""
+    w, x = _case(np.random.default_rng(k), ty, 64, k, many)
+    t = ctx.upload("blk.0.attn_q.weight", ty, k, 64, w)
+    x, y = torch.from_numpy(x).cuda(), torch.empty((many, 64), device="cuda")
+    long = torch.ones(1 << 28, device="cuda")  # work ahead of the calls, so that launching them takes no part
+    stream = torch.cuda.ExternalStream(ctx.stream)
+    torch.cuda.synchronize()
+    us = {}
+    for n in (few, many, few, many):
+        begin, end = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
+        with torch.cuda.stream(stream):
+            for _ in range(8):
+                long.mul_(1.0)
+            begin.record(stream)
+            for _ in range(40):
+                ctx.matmul_batch(t, x[:n], y[:n])
+            end.record(stream)
+        end.synchronize()
+        us[n] = min(us.get(n, 1e9), begin.elapsed_time(end) * 1e3 / 40)
+    t.free()
+    assert us[many] < 2.5 * us[few], us

@@ -1075,12 +1075,20 @@ size_t gemv_decode_rows_per_wg(uint32_t type, size_t rows, size_t cols) {
 // Token groups of 16 on the f64 matrix pipe: whole ones, a last one of 5 or
 // more beside them (5632->2048 at 21 / 117 tokens 38 -> 22 / 85 -> 68 us
 // against one token at a time for the rest; 3 more than 32 33 -> 37), and 6
-// or 9 tokens alone (11008->4096 at 6 57 -> 39, 2048->2048 at 6 / 12 6.5 /
-// 11.0 -> 8.7 / 8.9).
+// or 9 tokens alone (11008->4096 at 6 57 -> 39, 2048->2048 at 12 10.1 -> 8.5).
+// A group's time hardly depends on how many of its tokens and of the chip's
+// CUs it uses (one round of 256 workgroups, 16 rows each: 7 / 8 / 20 / 38 us at
+// K = 512 / 2048 / 5632 / 11008), the other kernel's on rows x tokens: where the
+// group needs a round of its own, those have to be worth it.  Groups / one at a
+// time (us): 9 tokens of 64 rows 6.8 / 2.6, 8.1 / 2.9, 19.7 / 4.9, 37 / 6.9 at
+// these K; 5632->1024 at 12 / 15 20 / 18, 21 / 23; 11008->1536 at 5 beside 32
+// 67 / 61; 2048->4096 at 5 beside 16 14.8 / 17.6.
 size_t gemv_q6_k_group_tokens(size_t rows, size_t cols, size_t batch) {
-    const size_t whole = batch / kQ6BTok, left = batch % kQ6BTok;
+    const size_t whole = batch / kQ6BTok, left = batch % kQ6BTok, wgs = (rows + kQ6BRows - 1) / kQ6BRows;
+    const auto rounds = [&](size_t groups) { return (wgs * groups + 255) / 256; };
     const size_t min_left = whole ? 5 : rows * cols >= (size_t{8} << 20) ? 6 : 9;
-    return left >= min_left ? batch : whole * kQ6BTok;
+    const size_t worth = (whole ? 12 << 10 : 16 << 10) * (rounds(whole + 1) - rounds(whole));
+    return left >= min_left && left * rows >= worth ? batch : whole * kQ6BTok;
 }
 
 hipError_t launch_gemv_q6_k(const uint8_t* W, const float* x, float* y, size_t rows, size_t cols, size_t batch,

@@ -58,7 +58,8 @@ def test_block_sums_where_they_pay_bitexact(ctx, oracle, ty, batch, k, n):
     test_block_sums_bitexact(ctx, oracle, ty, batch, k, n)
 
 
-@pytest.mark.parametrize("ty,few,many,k", [(synth.Q8_0, 2, 8, 8192), (synth.Q4_0, 2, 11, 8192)])
+@pytest.mark.parametrize("ty,few,many,k", [(synth.Q8_0, 2, 8, 8192), (synth.Q4_0, 2, 11, 8192), (synth.Q6_K, 2, 9, 5632),
+                                           (synth.Q6_K, 2, 15, 11008)])
 def test_few_rows_cost_by_their_tokens(ctx, ty, few, many, k):
     """A matrix of 64 rows leaves most of the chip idle, so more tokens of it cost next to nothing (1.0 to 1.1 times
     seen), unless they take a tile whose time is the same however full it is (4 to 5 times)."""

@@ -20,3 +20,12 @@ def test_token_groups(ctx, oracle, batch, k, n):
     for got in (ctx.matmul_batch(t, x), ctx.matmul_batch_v06(t, x, capi.MVH_ACT_Q8)):
         assert (np.abs(got - want) <= np.spacing(np.abs(want))).all()
     t.free()
+
+
+# rows and tokens on both sides of where a group of 9 or 6 tokens is worth a round of workgroups (16384 row-tokens), and
+# of 5 beside whole groups (12288): without another round of 256 workgroups, with one
+@pytest.mark.parametrize("batch,k,n", [(9, 512, 1820), (9, 512, 1821), (15, 256, 1092), (15, 256, 1093),
+                                       (6, 4096, 2730), (6, 4096, 2731), (8, 5632, 2048), (37, 256, 2100),
+                                       (37, 256, 2000), (21, 256, 2457), (21, 256, 2458)])
+def test_groups_worth_a_round(ctx, oracle, batch, k, n):
+    test_token_groups(ctx, oracle, batch, k, n)

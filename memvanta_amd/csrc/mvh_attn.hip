@@ -1034,12 +1034,18 @@ __global__ __launch_bounds__(kSM) void attn_softmax_rows_kernel(float* __restric
 // Value chains of a prefill chunk: workgroup (head h, 32-element slice of
 // head_dim, group of 32 query tokens); thread = (token b, 4 consecutive
 // elements), out[d] = fma(w_t, V_t[d], out[d]) over t = 0..pos0+b in order,
-// as in the reference (w_t the weights attn_scores_softmax_kernel wrote).  V rows come in 64-row tiles staged once in LDS for all
-// 32 tokens (the next tile's loads in flight while a tile is summed); the
-// rows past a token's last position (the chunk's later tokens, whatever they
-// hold) are left out, lane by lane, in the tiles that have any.  With q8 the output's
-// quantize_q8 blocks (one per token and slice) are written too, row-major or
-// in the prefill GEMM's operand order (q8_op).
+// as in the reference (w_t the weights attn_scores_softmax_kernel wrote).  V
+// rows come in 64-row tiles staged once in LDS for all 32 tokens (the next
+// tile's loads in flight while a tile is summed).  The rows past a token's last
+// position (the chunk's later tokens, whatever they hold) are left out: a wave
+// leaves out those that none of its 8 tokens sees and picks lane by lane where
+// they differ.  Only the last tiles of a chunk have such rows, so those have a
+// loop of their own: with the choice made lane by lane over whole tiles of one
+// loop a call took longer at every position (32 heads of 128, F16, 32 tokens at
+// 250 / 1000, one call after another: 25 / 50 us, 23 / 43 so; 2 tokens at 1900
+// 71, 59 so).  With q8 the output's quantize_q8 blocks (one per token and
+// slice) are written too, row-major or in the prefill GEMM's operand order
+// (q8_op).
 constexpr int kPV = 256;
 constexpr int kPVRows = 64;
 typedef _Float16 half4v __attribute__((ext_vector_type(4)));
@@ -1085,6 +1091,9 @@ __global__ __launch_bounds__(kPV) void attn_pv_chunk_kernel(int pos_arg, int B, 
     const int nmax = pos0 + min(B, b0 + 32);  // rows 0..nmax-1 are written (this chunk's included)
     const int tb = t >> 3, dq = (t & 7) * 4;  // chain: token b0 + tb, elements dq..dq+3 of the slice
     const int b = b0 + tb, nb = b < B ? pos0 + b + 1 : 0;
+    // the wave's 8 tokens: rows that all of them see, rows that any does
+    const int bw = b0 + 8 * __builtin_amdgcn_readfirstlane(t >> 6);
+    const int n_all = bw < B ? pos0 + bw + 1 : 0, n_some = bw < B ? pos0 + min(bw + 8, B) : 0;
     const int vr = t >> 2, vc = (t & 3) * 8;  // V staging: tile row vr, elements vc..vc+7
     const int ar_ = t >> 3, ac = (t & 7) * 8;  // weight staging: token b0 + ar_, tile rows ac..ac+7
     const int ab = b0 + ar_, nab = ab < B ? pos0 + ab + 1 : 0;
@@ -1110,8 +1119,42 @@ __global__ __launch_bounds__(kPV) void attn_pv_chunk_kernel(int pos_arg, int B, 
         }
     };
     float acc[4] = {0.f, 0.f, 0.f, 0.f};
-    fetch(0);
-    for (int r0 = 0; r0 < nmax; r0 += kPVRows) {
+    typedef typename PvRaw<KT>::T R;
+    auto ld = [&](int st, float4& w, R (&v)[4]) __attribute__((always_inline)) {  // rows 4 st .. of the tile
+        const int r = st << 2;
+        w = *reinterpret_cast<const float4*>(&s_at[tb][r]);
+#pragma unroll
+        for (int i = 0; i < 4; ++i) v[i] = *reinterpret_cast<const R*>(&s_v[r + i][dq]);
+    };
+    auto step = [&](float (&c)[4], const float4& w4, const R (&v)[4]) __attribute__((always_inline)) {
+        const float w[4] = {w4.x, w4.y, w4.z, w4.w};
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+#pragma unroll
+            for (int k = 0; k < 4; ++k) c[k] = fmaf(w[i], PvRaw<KT>::at(v[i], k), c[k]);
+    };
+    // nst whole 4-row steps with two register sets used in turn; every LDS read
+    // is unconditional (a step past the last re-reads the last one, unused) and
+    // the scheduling barriers keep the next set's reads ahead of the current
+    // set's fmas, so the wait counts never cover them
+    auto sum_steps = [&](auto nst) __attribute__((always_inline)) {
+        float4 wa, wb;
+        R va[4], vb[4];
+        ld(0, wa, va);
+        for (int st = 0; st < nst; st += 2) {
+            ld(min(st + 1, nst - 1), wb, vb);
+            __builtin_amdgcn_sched_barrier(0);
+            step(acc, wa, va);
+            __builtin_amdgcn_sched_barrier(0);
+            ld(min(st + 2, nst - 1), wa, va);
+            __builtin_amdgcn_sched_barrier(0);
+            float nx[4] = {acc[0], acc[1], acc[2], acc[3]};  // the odd step, kept when it exists
+            step(nx, wb, vb);
+#pragma unroll
+            for (int k = 0; k < 4; ++k) acc[k] = st + 1 < nst ? nx[k] : acc[k];
+        }
+    };
+    auto stage = [&](int r0) __attribute__((always_inline)) {  // tile r0 to LDS, the next one's loads issued
         if constexpr (KT == kKvF32) {
             *reinterpret_cast<uint4*>(&s_v[vr][vc]) = vreg[0];
             *reinterpret_cast<uint4*>(&s_v[vr][vc + 4]) = vreg[1];
@@ -1124,49 +1167,40 @@ __global__ __launch_bounds__(kPV) void attn_pv_chunk_kernel(int pos_arg, int B, 
         for (int j = 0; j < 8; ++j) s_at[ar_][ac + j] = areg[j];
         __syncthreads();
         if (r0 + kPVRows < nmax) fetch(r0 + kPVRows);
-        const int rows4 = min(kPVRows, (nmax - r0 + 3) & ~3);
-        // 4-row steps with two register sets used in turn; every LDS read is
-        // unconditional (a step past the last re-reads the last one, unused)
-        // and the scheduling barriers keep the next set's reads ahead of the
-        // current set's fmas, so the wait counts never cover them
-        typedef typename PvRaw<KT>::T R;
-        const int nst = rows4 >> 2;
-        auto ld = [&](int st, float4& w, R (&v)[4]) {
-            const int r = min(st, nst - 1) << 2;
-            w = *reinterpret_cast<const float4*>(&s_at[tb][r]);
+    };
+    fetch(0);
+    int r0 = 0;
+    for (; r0 + kPVRows <= pos0 + b0 + 1; r0 += kPVRows) {  // tiles that every token sees whole
+        stage(r0);
+        sum_steps(std::integral_constant<int, kPVRows / 4>{});
+        __syncthreads();
+    }
+    for (; r0 < nmax; r0 += kPVRows) {
+        stage(r0);
+        // the 4-row steps that all the wave's tokens see whole, and those that some of them see at all
+        const int nst = min(max(n_all - r0, 0) >> 2, kPVRows / 4);
+        const int nend = min((max(n_some - r0, 0) + 3) >> 2, kPVRows / 4);
+        if (nst) sum_steps(nst);
+        // the rest row by row, a token's own rows only: 8 consecutive tokens end within 3 steps
+        if (nst < nend) {
+            float4 w[3];
+            R v[3][4];
 #pragma unroll
-            for (int i = 0; i < 4; ++i) v[i] = *reinterpret_cast<const R*>(&s_v[r + i][dq]);
-        };
-        auto sum_tile = [&](auto masked) __attribute__((always_inline)) {
-            auto step = [&](float (&c)[4], int st, const float4& w4, const R (&v)[4]) {
-                const float w[4] = {w4.x, w4.y, w4.z, w4.w};
+            for (int j = 0; j < 3; ++j) ld(min(nst + j, nend - 1), w[j], v[j]);
 #pragma unroll
-                for (int i = 0; i < 4; ++i)
+            for (int j = 0; j < 3; ++j) {
+                const float wj[4] = {w[j].x, w[j].y, w[j].z, w[j].w};
+#pragma unroll
+                for (int i = 0; i < 4; ++i) {
+                    const bool mine = nst + j < nend && r0 + 4 * (nst + j) + i < nb;
 #pragma unroll
                     for (int k = 0; k < 4; ++k) {
-                        const float s = fmaf(w[i], PvRaw<KT>::at(v[i], k), c[k]);
-                        c[k] = !decltype(masked)::value || r0 + 4 * st + i < nb ? s : c[k];
+                        const float s = fmaf(wj[i], PvRaw<KT>::at(v[j][i], k), acc[k]);
+                        acc[k] = mine ? s : acc[k];
                     }
-            };
-            float4 wa, wb;
-            R va[4], vb[4];
-            ld(0, wa, va);
-            for (int st = 0; st < nst; st += 2) {
-                ld(st + 1, wb, vb);
-                __builtin_amdgcn_sched_barrier(0);
-                step(acc, st, wa, va);
-                __builtin_amdgcn_sched_barrier(0);
-                ld(st + 2, wa, va);
-                __builtin_amdgcn_sched_barrier(0);
-                float nx[4] = {acc[0], acc[1], acc[2], acc[3]};  // the odd step, kept when it exists
-                step(nx, st + 1, wb, vb);
-#pragma unroll
-                for (int k = 0; k < 4; ++k) acc[k] = st + 1 < nst ? nx[k] : acc[k];
+                }
             }
-        };
-        // a tile with rows that some of the 32 tokens do not see, or one without
-        if (r0 + kPVRows > pos0 + b0 + 1) sum_tile(std::true_type{});
-        else sum_tile(std::false_type{});
+        }
         __syncthreads();
     }
     if (b >= B) return;  // whole 8-lane groups (one token) leave together

@@ -69,21 +69,21 @@ def test_buffers_of_a_model_that_never_joins(tiny):
 
 
 @pytest.mark.parametrize("kv_type", [capi.MVH_KV_F32, capi.MVH_KV_F16])
-@pytest.mark.parametrize("B", [31, 40])
-def test_later_rows_do_not_reach_earlier_tokens(ctx, kv_type, B):
+@pytest.mark.parametrize("B,pos,last", [(31, 70, 3), (40, 70, 3), (40, 100, 9), (33, 0, 1), (13, 55, 5)])
+def test_later_rows_do_not_reach_earlier_tokens(ctx, kv_type, B, pos, last):
     """V rows past a token's position may hold anything: an infinity there leaves the token's output as it was."""
     rng = np.random.default_rng(B)
-    n_head, hd, pos = 4, 64, 70
+    n_head, hd = 4, 64
     k, v = (rng.standard_normal((pos + B, n_head * hd), dtype=np.float32) for _ in range(2))
     q = rng.standard_normal((B, n_head * hd), dtype=np.float32)
     outs = []
     for far in (0.5, np.inf):
-        v[pos + B - 3:] = far
+        v[pos + B - last:] = far
         kv = ctx.kv_cache(1, n_head * hd, 16, 256, kv_type=kv_type)
         kv.write(0, 0, k, v)
         outs.append(kv.attn_batch(0, q, pos, B, n_head, n_head, hd).copy())
         kv.close()
-    a, b = (o[: B - 3].view(np.uint32) for o in outs)
+    a, b = (o[: B - last].view(np.uint32) for o in outs)
     assert (a == b).all()
 
 

@@ -1180,25 +1180,25 @@ __global__ __launch_bounds__(kPV) void attn_pv_chunk_kernel(int pos_arg, int B, 
         // the 4-row steps that all the wave's tokens see whole, and those that some of them see at all
         const int nst = min(max(n_all - r0, 0) >> 2, kPVRows / 4);
         const int nend = min((max(n_some - r0, 0) + 3) >> 2, kPVRows / 4);
-        if (nst) sum_steps(nst);
-        // the rest row by row, a token's own rows only: 8 consecutive tokens end within 3 steps
-        if (nst < nend) {
-            float4 w[3];
-            R v[3][4];
+        // the rest, a token's own rows only: 8 consecutive tokens end within 3 steps (read ahead of the others)
+        float4 w[3];
+        R v[3][4];
+        if (nst < nend)
 #pragma unroll
             for (int j = 0; j < 3; ++j) ld(min(nst + j, nend - 1), w[j], v[j]);
+        __builtin_amdgcn_sched_barrier(0);
+        if (nst) sum_steps(nst);
+        if (nst < nend) {
 #pragma unroll
             for (int j = 0; j < 3; ++j) {
-                const float wj[4] = {w[j].x, w[j].y, w[j].z, w[j].w};
+                float wj[4] = {w[j].x, w[j].y, w[j].z, w[j].w};
 #pragma unroll
-                for (int i = 0; i < 4; ++i) {
+                for (int i = 0; i < 4; ++i) {  // a row left out: fma(-0, +0, acc) is acc, whatever its sign
                     const bool mine = nst + j < nend && r0 + 4 * (nst + j) + i < nb;
-#pragma unroll
-                    for (int k = 0; k < 4; ++k) {
-                        const float s = fmaf(wj[i], PvRaw<KT>::at(v[j][i], k), acc[k]);
-                        acc[k] = mine ? s : acc[k];
-                    }
+                    wj[i] = mine ? wj[i] : -0.0f;
+                    v[j][i] = mine ? v[j][i] : R{};
                 }
+                step(acc, make_float4(wj[0], wj[1], wj[2], wj[3]), v[j]);
             }
         }
         __syncthreads();

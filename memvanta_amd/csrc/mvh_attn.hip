@@ -1553,6 +1553,17 @@ const bool kScoresTile = [] {
     return !(e && atoi(e) == 0);
 }();
 
+// Whether F16 scores take K tiles (head_dim 128 / 64, 8 tokens or more).  Up to
+// 32 tokens always: several streams' chunks share the chip better that way.
+// Beyond, where the (head, row) pairs are enough: a call of few is as long as
+// one workgroup's tile, while the per-(head, token) kernel's time is its pairs.
+// attn_batch, that kernel / tiles (us, 32 heads): of 128 40 tokens at 0 / 250 /
+// 480 8 / 16, 24 / 23, 37 / 30, 64 at 64 / 130 15 / 18, 22 / 21, 128 at 0 / 30
+// 19 / 20, 25 / 24; of 64 40 at 250 / 480 19 / 19.4, 28 / 24, 128 at 30 / 64 17 / 18, 19 / 18.
+bool scores_in_tiles(size_t pos, size_t B, size_t n_head, size_t hd) {
+    return B <= 32 || n_head * B * (2 * pos + B) >= (hd == 128 ? size_t{640} << 10 : size_t{800} << 10);
+}
+
 template <int KT>
 hipError_t attn_prefill_typed(const void* const* pt_k, const void* const* pt_v, const float* q, size_t q_pitch,
                               float* a_scratch, float* out, int8_t* q8, float* q8d, bool q8_op, const int* d_pos,
@@ -1560,9 +1571,9 @@ hipError_t attn_prefill_typed(const void* const* pt_k, const void* const* pt_v, 
                               size_t kv_dim, size_t page_tokens, hipStream_t st) {
     const int group = static_cast<int>(n_head / n_head_kv);
     const int pitch = static_cast<int>(max_pos);  // weight row pitch >= last position + 1
-    if (kScoresTile && KT == kKvF16 && !d_pos && B >= 8 && (hd == 128 || hd == 64) && q_pitch % 4 == 0 &&
-        (reinterpret_cast<uintptr_t>(q) & 15) == 0) {
-        // F16 chunks of 8 tokens or more, q rows 16-byte aligned: K staged once per (head, 64-row block, 32 tokens)
+    if (kScoresTile && KT == kKvF16 && !d_pos && B >= 8 && (hd == 128 || hd == 64) &&
+        scores_in_tiles(pos, B, n_head, hd) && q_pitch % 4 == 0 && (reinterpret_cast<uintptr_t>(q) & 15) == 0) {
+        // F16 chunks, q rows 16-byte aligned: K staged once per (head, 64-row block, 32 tokens)
         const dim3 gs(static_cast<unsigned>(n_head), static_cast<unsigned>((pos + B + kTR - 1) / kTR),
                       static_cast<unsigned>((B + 31) / 32));
         if (hd == 128)

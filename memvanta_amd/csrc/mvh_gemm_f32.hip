@@ -325,10 +325,54 @@ void chain_one(const uint8_t* W, const float* x, float* y, int N, int nb, int B,
     batch_chain_kernel<TYPE, E, R, TG, D, ALIGNED><<<grid, kT, 0, st>>>(W, x, y, N, nb, B);
 }
 
+// The same chains of rows of up to 3 blocks, a thread per (row, token): a
+// unit of the matrix-pipe kernel is 8 blocks of work however few a row has.
+// That kernel / this one at 512 tokens of 11008 rows (us): Q4_0 K = 32 / 64 /
+// 96 75 / 28, 75 / 44, 76 / 66, Q8_0 95 / 33, 98 / 61, 96 / 103, at 11 tokens
+// Q8_0 K = 96 9.9 / 8.6; even at 128.
+constexpr int kShortK = 96;
+template <uint32_t TYPE>
+__global__ __launch_bounds__(kT) void batch_short_kernel(const uint8_t* __restrict__ W, const float* __restrict__ x,
+                                                          float* __restrict__ y, int N, int nb) {
+    constexpr int kQ = TYPE == kQ4_0 ? 4 : 8;  // dwords of quants in a block
+    __shared__ float s_x[kShortK];
+    const int K = nb * 32;
+    const float* xt = x + static_cast<size_t>(blockIdx.y) * K;
+    if (static_cast<int>(threadIdx.x) < K) s_x[threadIdx.x] = xt[threadIdx.x];
+    __syncthreads();
+    const int r = blockIdx.x * kT + threadIdx.x;
+    if (r >= N) return;
+    const uint16_t* src = reinterpret_cast<const uint16_t*>(W + static_cast<size_t>(r) * nb * Fmt<TYPE>::kB);
+    float t[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+    for (int b = 0; b < nb; ++b, src += Fmt<TYPE>::kB / 2) {
+        uint32_t q[kQ];
+#pragma unroll
+        for (int k = 0; k < kQ; ++k) q[k] = src[1 + 2 * k] | static_cast<uint32_t>(src[2 + 2 * k]) << 16;
+        const float d = h2f(src[0]);
+#pragma unroll
+        for (int k = 0; k < 8; ++k) {  // elements 4k .. 4k + 3
+            float a[4];
+            if constexpr (TYPE == kQ4_0) weights<TYPE, 4>((q[k & 3] ^ 0x88888888u) >> (k < 4 ? 0 : 4), d * 16.0f, a);
+            else weights<TYPE, 4>(q[k], d, a);
+#pragma unroll
+            for (int i = 0; i < 4; ++i) t[4 * (k & 1) + i] = fmaf(a[i], s_x[32 * b + 4 * k + i], t[4 * (k & 1) + i]);
+        }
+    }
+    float s = t[0];
+#pragma unroll
+    for (int e = 1; e < 8; ++e) s = s + t[e];
+    y[static_cast<size_t>(blockIdx.y) * N + r] = s;
+}
+
 template <uint32_t TYPE>
 hipError_t launch_chain(const uint8_t* W, const float* x, float* y, size_t rows, size_t cols, size_t batch,
                         hipStream_t st) {
     const int N = static_cast<int>(rows), nb = static_cast<int>(cols / 32), B = static_cast<int>(batch);
+    if (cols <= kShortK && batch <= 65535) {  // grid y: tokens
+        const dim3 grid(static_cast<unsigned>((rows + kT - 1) / kT), static_cast<unsigned>(batch));
+        batch_short_kernel<TYPE><<<grid, kT, 0, st>>>(W, x, y, N, nb);
+        return hipGetLastError();
+    }
     const bool aligned = cols % 256 == 0 && (reinterpret_cast<uintptr_t>(W) & 15) == 0;
     if (!aligned) {
         chain_one<TYPE, 2, 1, 1, 2, false>(W, x, y, N, nb, B, st);

@@ -32,6 +32,46 @@ def test_chain_tiles_bitexact(ctx, oracle, ty, batch, k, n):
     t.free()
 
 
+# rows of up to three blocks have a kernel of their own, four and more the matrix pipe; rows at the edges of its 256
+@pytest.mark.parametrize("ty", [synth.Q4_0, synth.Q8_0])
+@pytest.mark.parametrize("batch,k,n", [(4, 32, 256), (8, 32, 257), (12, 64, 1000), (16, 96, 255), (4, 96, 1),
+                                       (24, 128, 257), (8, 160, 300)])
+def test_short_rows_bitexact(ctx, oracle, ty, batch, k, n):
+    test_chain_tiles_bitexact(ctx, oracle, ty, batch, k, n)
+
+
+def _us(call, ctx):
+    """Time of a call: 40 of them queued behind other work, so that launching them takes no part."""
+    long = torch.ones(1 << 28, device="cuda")
+    stream = torch.cuda.ExternalStream(ctx.stream)
+    torch.cuda.synchronize()
+    best = 1e9
+    for _ in range(2):
+        begin, end = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
+        with torch.cuda.stream(stream):
+            for _ in range(8):
+                long.mul_(1.0)
+            begin.record(stream)
+            for _ in range(40):
+                call()
+            end.record(stream)
+        end.synchronize()
+        best = min(best, begin.elapsed_time(end) * 1e3 / 40)
+    return best
+
+
+def test_short_rows_cost_by_their_length(ctx):
+    """A row of one block costs well under half of one of four (0.4 times seen), not as much as a whole 8-block unit."""
+    us = {}
+    for k in (32, 128):
+        w, x = _case(np.random.default_rng(k), synth.Q4_0, 11008, k, 512)
+        t = ctx.upload("blk.0.attn_q.weight", synth.Q4_0, k, 11008, w)
+        x, y = torch.from_numpy(x).cuda(), torch.empty((512, 11008), device="cuda")
+        us[k] = _us(lambda: ctx.matmul_batch_v06(t, x, capi.MVH_ACT_REF, y), ctx)
+        t.free()
+    assert us[32] < 0.6 * us[128], us
+
+
 # tokens: the first batch on this kernel, one short of and past its 16-token tiles; rows at the edges of 16 and 32, on
 # both sides of the 512-workgroup line; K: half a round of 16 blocks, one, one and a half, many
 @pytest.mark.parametrize("ty", [synth.Q4_0, synth.Q8_0])
@@ -66,20 +106,6 @@ def test_few_rows_cost_by_their_tokens(ctx, ty, few, many, k):
     w, x = _case(np.random.default_rng(k), ty, 64, k, many)
     t = ctx.upload("blk.0.attn_q.weight", ty, k, 64, w)
     x, y = torch.from_numpy(x).cuda(), torch.empty((many, 64), device="cuda")
-    long = torch.ones(1 << 28, device="cuda")  # work ahead of the calls, so that launching them takes no part
-    stream = torch.cuda.ExternalStream(ctx.stream)
-    torch.cuda.synchronize()
-    us = {}
-    for n in (few, many, few, many):
-        begin, end = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
-        with torch.cuda.stream(stream):
-            for _ in range(8):
-                long.mul_(1.0)
-            begin.record(stream)
-            for _ in range(40):
-                ctx.matmul_batch(t, x[:n], y[:n])
-            end.record(stream)
-        end.synchronize()
-        us[n] = min(us.get(n, 1e9), begin.elapsed_time(end) * 1e3 / 40)
+    us = {n: _us(lambda: ctx.matmul_batch(t, x[:n], y[:n]), ctx) for n in (few, many)}
     t.free()
     assert us[many] < 2.5 * us[few], us

@@ -962,12 +962,13 @@ static hipError_t launch_f32act(const uint8_t* W, const float* x, float* y, size
 // they are even or ahead (4096x4096 Q4_0 at 2 / 3 / 4 tokens 11.6 / 15.6 / 18.3
 // against 17.8 us).  8 tokens, matrix pipe / those (us, Q8_0): 512->64 3.7 / 8.6,
 // 2048->64 9.6 / 10.1; 4096->64 / 768 / 2048 18 / 8.6, 18 / 11.6, 18 / 20;
-// 8192->64 / 1024 / 1536 34 / 7, 34 / 30, 34 / 41; 11008->1024 46 / 79.  4..7
-// tokens beyond K = 4608 want more rows (8192->1536 at 6 34 / 32).
-static bool enough_for_blocksum(size_t rows, size_t cols, size_t batch) {
+// 8192->64 / 1024 / 1536 34 / 7, 34 / 30, 34 / 41; 11008->1024 46 / 79; Q4_0
+// costs those less (4096->2048 at 7 tokens 18 / 15, Q8_0 18 / 19).  4..7 tokens
+// beyond K = 4608 want more rows (8192->1536 at 6 34 / 32).
+static bool enough_for_blocksum(uint32_t type, size_t rows, size_t cols, size_t batch) {
     const size_t work = rows * batch;
     if (cols <= 2048) return true;
-    if (cols <= 4608) return work > (cols <= 3072 ? 5 << 10 : 12 << 10);
+    if (cols <= 4608) return work > (cols <= 3072 ? 5 << 10 : type == kQ4_0 ? 14 << 10 : 12 << 10);
     return work >= 8 << 10 && (batch >= 8 || rows >= 4096);
 }
 
@@ -1014,7 +1015,7 @@ static hipError_t launch_f32act_any(const uint8_t* W, const float* x, float* y, 
         return hipGetLastError();
     }
     if constexpr (TYPE == kQ4_0 || TYPE == kQ8_0) {
-        if (batch >= 4 && enough_for_blocksum(rows, cols, batch) && batch_blocksum_ok(TYPE, W, cols))
+        if (batch >= 4 && enough_for_blocksum(TYPE, rows, cols, batch) && batch_blocksum_ok(TYPE, W, cols))
             return launch_batch_blocksum(TYPE, W, x, y, rows, cols, batch, st);
     }
     return launch_f32act<TYPE>(W, x, y, rows, cols, batch, st);

@@ -1043,9 +1043,10 @@ __global__ __launch_bounds__(kSM) void attn_softmax_rows_kernel(float* __restric
 // loop of their own: with the choice made lane by lane over whole tiles of one
 // loop a call took longer at every position (32 heads of 128, F16, 32 tokens at
 // 250 / 1000, one call after another: 25 / 50 us, 23 / 43 so; 2 tokens at 1900
-// 71, 59 so).  With q8 the output's quantize_q8 blocks (one per token and
-// slice) are written too, row-major or in the prefill GEMM's operand order
-// (q8_op).
+// 71, 59 so).  Eight waves a SIMD (F32 five) for calls of several streams side by
+// side: three contexts' chunks of 8 tokens at 512 11.5 us a call before, 10.3 so.
+// With q8 the output's quantize_q8 blocks (one per token and slice) are written
+// too, row-major or in the prefill GEMM's operand order (q8_op).
 constexpr int kPV = 256;
 constexpr int kPVRows = 64;
 typedef _Float16 half4v __attribute__((ext_vector_type(4)));
@@ -1076,7 +1077,7 @@ struct PvRaw<kKvQ8> {
     }
 };
 template <int KT>
-__global__ __launch_bounds__(kPV) void attn_pv_chunk_kernel(int pos_arg, int B, int n_head, int group, int hd,
+__global__ __launch_bounds__(kPV, KT == kKvF32 ? 5 : 8) void attn_pv_chunk_kernel(int pos_arg, int B, int n_head, int group, int hd,
                                                             int kv_dim, int page_tokens, int pitch,
                                                             const void* const* __restrict__ pt_v,
                                                             const float* __restrict__ a, const int* __restrict__ d_pos,
@@ -1180,26 +1181,29 @@ __global__ __launch_bounds__(kPV) void attn_pv_chunk_kernel(int pos_arg, int B, 
         // the 4-row steps that all the wave's tokens see whole, and those that some of them see at all
         const int nst = min(max(n_all - r0, 0) >> 2, kPVRows / 4);
         const int nend = min((max(n_some - r0, 0) + 3) >> 2, kPVRows / 4);
-        // the rest, a token's own rows only: 8 consecutive tokens end within 3 steps (read ahead of the others)
-        float4 w[3];
-        R v[3][4];
-        if (nst < nend)
-#pragma unroll
-            for (int j = 0; j < 3; ++j) ld(min(nst + j, nend - 1), w[j], v[j]);
-        __builtin_amdgcn_sched_barrier(0);
         if (nst) sum_steps(nst);
-        if (nst < nend) {
-#pragma unroll
-            for (int j = 0; j < 3; ++j) {
-                float wj[4] = {w[j].x, w[j].y, w[j].z, w[j].w};
+        if (nst < nend) {  // the rest, a token's own rows only: 8 consecutive tokens end within 3 steps
+            auto own = [&](int st, float4& w4, R (&v)[4]) __attribute__((always_inline)) {
+                float w[4] = {w4.x, w4.y, w4.z, w4.w};
 #pragma unroll
                 for (int i = 0; i < 4; ++i) {  // a row left out: fma(-0, +0, acc) is acc, whatever its sign
-                    const bool mine = nst + j < nend && r0 + 4 * (nst + j) + i < nb;
-                    wj[i] = mine ? wj[i] : -0.0f;
-                    v[j][i] = mine ? v[j][i] : R{};
+                    const bool mine = st < nend && r0 + 4 * st + i < nb;
+                    w[i] = mine ? w[i] : -0.0f;
+                    v[i] = mine ? v[i] : R{};
                 }
-                step(acc, make_float4(wj[0], wj[1], wj[2], wj[3]), v[j]);
-            }
+                step(acc, make_float4(w[0], w[1], w[2], w[3]), v);
+            };
+            float4 wa, wb;
+            R va[4], vb[4];
+            ld(nst, wa, va);
+            ld(min(nst + 1, nend - 1), wb, vb);
+            __builtin_amdgcn_sched_barrier(0);
+            own(nst, wa, va);
+            __builtin_amdgcn_sched_barrier(0);
+            ld(min(nst + 2, nend - 1), wa, va);
+            __builtin_amdgcn_sched_barrier(0);
+            own(nst + 1, wb, vb);
+            own(nst + 2, wa, va);
         }
         __syncthreads();
     }

@@ -384,7 +384,9 @@ hipError_t launch_chain(const uint8_t* W, const float* x, float* y, size_t rows,
     // at 512); the workgroups of the busiest of the 256 CUs count.  Small tiles
     // keep every CU busy where there are few rows (4096x4096 at 32 tokens:
     // 16x32 17.5 us, 32x32 28 us), larger ones read the activations less often
-    // (at 512 tokens: 32x32 176 us, 16x32 208 us, 16x16 220 us).
+    // (at 512 tokens: 32x32 176 us, 16x32 208 us, 16x16 220 us).  All of it is
+    // Q4_0's: a Q8_0 workgroup takes 83 KB of LDS at 32x32 and 92 at 48x32, so
+    // a CU has one of them and not two.
     struct Tile {
         int rows, toks;
         float alone, shared;

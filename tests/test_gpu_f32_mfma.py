@@ -92,8 +92,9 @@ def test_block_sums_bitexact(ctx, oracle, ty, batch, k, n):
 # to 3072, 12 K (Q8_0) or 14 K (Q4_0) up to 4608, 8 K beyond (there with 4096 rows or 8 tokens)
 @pytest.mark.parametrize("ty", [synth.Q4_0, synth.Q8_0])
 @pytest.mark.parametrize("batch,k,n", [(4, 2048, 33), (4, 2304, 1280), (4, 2304, 1281), (5, 3072, 1025),
-                                       (8, 3328, 1536), (8, 3328, 1537), (7, 3328, 2048), (7, 3328, 2049), (16, 4608, 769), (8, 4864, 1023),
-                                       (8, 4864, 1024), (7, 8192, 1200), (4, 5120, 4096), (17, 8192, 600)])
+                                       (8, 3328, 1536), (8, 3328, 1537), (7, 3328, 2048), (7, 3328, 2049),
+                                       (16, 4608, 769), (8, 4864, 1023), (8, 4864, 1024), (7, 8192, 1200),
+                                       (4, 5120, 4096), (17, 8192, 600)])
 def test_block_sums_where_they_pay_bitexact(ctx, oracle, ty, batch, k, n):
     test_block_sums_bitexact(ctx, oracle, ty, batch, k, n)
 
